@@ -340,63 +340,55 @@ __device__ __forceinline__ d2 shakhov_eq(const Consts &C, d4 p, d2 Q, d2 uv, int
 __device__ __forceinline__ double van_leer(double s1, double s2) {
     return (ocl_sign(s1) + ocl_sign(s2)) * (fabs(s1) * fabs(s2)) / (fabs(s1) + fabs(s2) + 1e-16);
 }
-// WENO5 slope of both components (g, h) (clFunctions.c:268-312), written
-// in the first differences d_k = s_k - s_{k-1}:
-//   smoothness  12 b_0 = 13 (d2 - d1)^2 + 3 (3 d2 - d1)^2
-//               12 b_1 = 13 (d3 - d2)^2 + 3 (d2 + d3)^2
-//               12 b_2 = 13 (d4 - d3)^2 + 3 (3 d3 - d4)^2
-//   candidates  f_0 - s2 = -d1/3 + 5 d2/6,  f_1 - s2 = d2/6 + d3/3,
-//               f_2 - s2 = 2 d3/3 - d4/6
-// with eps scaled by 12 alongside (the weights only see the ratios), so that
-// (f_L - s2) is formed without cancelling against s2.  The nonlinear weights
-// a_k = d_k / (eps + b_k)^2 are written 1 / e_k^2 with e_k = 12 (eps + b_k)
-// / sqrt(d_k): the linear weights d = (0.1, 0.6, 0.3) ride in the constants
-// of e_k, which is one multiply and two FMAs from the differences.  They
-// enter only through sum(a_k (f_k - s2)) / sum(a_k): in double both sums are
-// scaled by prod_k e_k^2, leaving one quotient per component, and the two
-// quotients share one reciprocal.  (In float that product can underflow:
-// the FP32 form takes reciprocal estimates of the weights instead.)
-// e_k = A_k u_k^2 + B_k v_k^2 + E_k with A_k = 13 / sqrt(d_k), B_k = 3 / sqrt(d_k), E_k = 1.2e-15 / sqrt(d_k)
+// WENO5 (clFunctions.c:268-312), written in the first differences d_k = s_k -
+// s_{k-1} and the second ones u0 = d2 - d1, u1 = d3 - d2, n2 = d3 - d4:
+//   smoothness  12 b_0 = 13 (d2 - d1)^2 + 3 (3 d2 - d1)^2 = 4 (u0 (4 u0 + 3 d2) + 3 d2^2)
+//               12 b_1 = 13 (d3 - d2)^2 + 3 (d2 + d3)^2   = 4 (u1 (4 u1 + 3 d2) + 3 d2^2)
+//               12 b_2 = 13 (d4 - d3)^2 + 3 (3 d3 - d4)^2 = 4 (n2 (4 n2 + 3 d3) + 3 d3^2)
+//   candidates  6 (f_0 - s2) = 5 d2 - 2 d1 = 3 d2 + 2 u0
+//               6 (f_1 - s2) = d2 + 2 d3   = 3 d2 + 2 u1
+//               6 (f_2 - s2) = 4 d3 - d4   = 3 d3 + n2
+// with 3 d2, 3 d3 and 3 d2^2 + eps', 3 d3^2 + eps' shared (eps' = 3 eps: the
+// weights only see ratios of b_k + eps).  The quadratic forms are positive
+// definite; their largest cancellation (u against d) costs a factor 2.5.
+// The face value is s2 + q / 6 and the slope q / (6 dist) with
+// q = sum(a_k 6 (f_k - s2)) / sum(a_k), a_k = d_k / (eps + b_k)^2 and
+// d = (1, 6, 3) / 10, so neither needs the distance in the velocity loop.
+// Both sums are scaled by prod_k (eps + b_k)^2, leaving one quotient per
+// component, and the two quotients of a (g, h) pair share one reciprocal.
+constexpr double kWenoEps = 3e-16;
+// The FP32 form (ugks_fused.hip), where that product can underflow, takes
+// e_k = A_k u_k^2 + B_k v_k^2 + E_k, A_k = 13 / sqrt(d_k), B_k = 3 / sqrt(d_k), E_k = 1.2e-15 / sqrt(d_k)
 constexpr double kWA0 = 41.10960958218893, kWB0 = 9.486832980505138, kWE0 = 3.794733192202055e-15;
 constexpr double kWA1 = 16.782927833565473, kWB1 = 3.8729833462074166, kWE1 = 1.5491933384829667e-15;
 constexpr double kWA2 = 23.7346441585572, kWB2 = 5.477225575051661, kWE2 = 2.1908902300206646e-15;
 struct WenoParts { double num, den; };
 __device__ __forceinline__ WenoParts weno5_parts(double s0, double s1, double s2, double s3, double s4) {
     const double d1 = s1 - s0, d2 = s2 - s1, d3 = s3 - s2, d4 = s4 - s3;
-    const double u0 = d2 - d1, v0 = 3.0 * d2 - d1;
-    const double u1 = d3 - d2, v1 = d2 + d3;
-    const double u2 = d4 - d3, v2 = 3.0 * d3 - d4;
-    const double e0 = fma(kWA0 * u0, u0, fma(kWB0 * v0, v0, kWE0));
-    const double e1 = fma(kWA1 * u1, u1, fma(kWB1 * v1, v1, kWE1));
-    const double e2 = fma(kWA2 * u2, u2, fma(kWB2 * v2, v2, kWE2));
+    const double u0 = d2 - d1, u1 = d3 - d2, n2 = d3 - d4, m2 = 3.0 * d2, m3 = 3.0 * d3;
+    const double b2 = fma(m2, d2, kWenoEps), b3 = fma(m3, d3, kWenoEps);
+    const double e0 = fma(u0, fma(4.0, u0, m2), b2), e1 = fma(u1, fma(4.0, u1, m2), b2), e2 = fma(n2, fma(4.0, n2, m3), b3);
+    const double c0 = fma(2.0, u0, m2), c1 = fma(2.0, u1, m2), c2 = m3 + n2;
     const double q0 = e0 * e0, q1 = e1 * e1, q2 = e2 * e2;
-    const double p0 = q1 * q2, p1 = q0 * q2, p2 = q0 * q1;
-    // (f_k - s2)
-    const double c0 = (-1.0 / 3.0) * d1 + (5.0 / 6.0) * d2;
-    const double c1 = (1.0 / 6.0) * d2 + (1.0 / 3.0) * d3;
-    const double c2 = (2.0 / 3.0) * d3 - (1.0 / 6.0) * d4;
+    const double p0 = q1 * q2, p1 = (6.0 * q0) * q2, p2 = (3.0 * q0) * q1;
     return WenoParts{p0 * c0 + p1 * c1 + p2 * c2, (p0 + p1) + p2};
 }
-// the two slopes (f_L - s2) / dist of a (g, h) stencil
-__device__ __forceinline__ void weno5_slope_pair(double g0, double g1, double g2, double g3, double g4, double h0,
-                                                 double h1, double h2, double h3, double h4, double rdx, double &sgx,
-                                                 double &sgy) {
+// q of both components of a (g, h) stencil
+__device__ __forceinline__ void weno5_q_pair(double g0, double g1, double g2, double g3, double g4, double h0, double h1,
+                                             double h2, double h3, double h4, double &qg, double &qh) {
     const WenoParts a = weno5_parts(g0, g1, g2, g3, g4);
     const WenoParts b = weno5_parts(h0, h1, h2, h3, h4);
-    // 1 / (den_a den_b) from the hardware estimate and two Newton steps; the
-    // dens are >= (1.2e-15)^4 and far below overflow, so is their product
+    // 1 / (den_a den_b) from the hardware estimate and one Newton step; the
+    // residual correction of each quotient squares what error is left.  The
+    // dens are >= 10 (3e-16)^4 and far below overflow, so is their product.
     const double D = a.den * b.den;
     double r = __builtin_amdgcn_rcp(D);
-    double e = fma(-D, r, 1.0);
-    r = fma(r, e, r);
-    e = fma(-D, r, 1.0);
-    r = fma(r, e, r);
+    r = fma(r, fma(-D, r, 1.0), r);
     const double ra = r * b.den, rb = r * a.den;     // 1 / den_a, 1 / den_b
-    double qa = a.num * ra, qb = b.num * rb;
-    qa = fma(ra, fma(-a.den, qa, a.num), qa);        // one residual correction each
-    qb = fma(rb, fma(-b.den, qb, b.num), qb);
-    sgx = qa * rdx;
-    sgy = qb * rdx;
+    qg = a.num * ra;
+    qh = b.num * rb;
+    qg = fma(ra, fma(-a.den, qg, a.num), qg);
+    qh = fma(rb, fma(-b.den, qh, b.num), qh);
 }
 // minmod + NND (clFunctions.c:320-352), one component
 __device__ __forceinline__ double minmod(double a, double b) {
@@ -574,14 +566,14 @@ __device__ __forceinline__ void wave_sum4(double (&a)[4]) {
 #pragma unroll
     for (int q = 0; q < 4; q++) a[q] = lane_d(r, 16 * q);
 }
-// Totals of a[0..15] over the wavefront: every lane of row r gets the totals
-// of a[4r .. 4r+3] in t[0..3].
-__device__ __forceinline__ void wave_sum16_rows(const double (&a)[16], double (&t)[4]) {
-    double s[8];
+// Totals of a[0..4N-1] over the wavefront: every lane of row r gets the totals
+// of a[N r .. N r + N - 1] in t[0..N-1].
+template <int N> __device__ __forceinline__ void wave_sum_rows(const double (&a)[4 * N], double (&t)[N]) {
+    double s[2 * N];
 #pragma unroll
-    for (int k = 0; k < 8; k++) s[k] = fold32(a[k], a[k + 8]);      // value k (lanes 0-31), k + 8 (32-63)
+    for (int k = 0; k < 2 * N; k++) s[k] = fold32(a[k], a[k + 2 * N]);    // value k (lanes 0-31), k + 2N (32-63)
 #pragma unroll
-    for (int k = 0; k < 4; k++) t[k] = row_sum(fold16(s[k], s[k + 4]));   // value k + 4 r in row r
+    for (int k = 0; k < N; k++) t[k] = row_sum(fold16(s[k], s[k + N]));   // value k + N r in row r
 }
 
 }  // namespace ugks

@@ -6,9 +6,7 @@
 //
 //   k_faceA   one wavefront per interior face (S and W faces of all blocks):
 //             reconstruction (iFace) and the raw velocity moments of the face
-//             values (getFaceCons and the sums calcFaceQ needs), of the left
-//             and right cells (getAL/getAR) and of the owner cell (calcQ, on
-//             S faces).
+//             values (getFaceCons and the sums calcFaceQ needs).
 //   k_faceS   one thread per interior face: primary variables, slopes and
 //             time slope (getPLR/initMacroFlux), face heat flux (calcFaceQ)
 //             and the equilibrium part of the macro flux, folded into the
@@ -18,8 +16,9 @@
 //   k_wall    one workgroup per diffuse/adsorbing wall face: reconstruction,
 //             accommodatingWallDist or adsorbingWall_P1 + S/D_P2, wallFlux,
 //             wallMassEnergyFluxes.
-//   k_update  one wavefront per cell: updateMacro + UGKS_update and the
-//             cell's moments for the next step's left/right face states.
+//   k_update  one wavefront per cell: updateMacro + UGKS_update, the cell's
+//             moments for the next step's left/right face states (getAL/getAR)
+//             and its heat flux for the next update (calcQ).
 //   k_dt      one thread per cell: clFindDT and the per-block maximum.
 //   k_dtfin   one workgroup: the global time step with the reference's growth
 //             limit (ugks_sim.py:285-311, applied as one_step does, :430-446).
@@ -71,6 +70,7 @@ struct FBlock {
     int nS, nSj, ob_S, ob_W, nWi, wl;       // interior-face counts and offsets
     int flipidx[4];                         // exchange row flip from the corner check
     int cs;                                 // case of this block (its time-step state)
+    d2 *qnext;                              // [ni][nj] heat flux of f about macro, for the next update
     d4 *cmom;                               // [NI][NJ] moments of f per cell (all cells, ghosts included)
 };
 
@@ -154,29 +154,29 @@ template <int N> __device__ __forceinline__ void block_sum(double (&a)[N], doubl
 // ---- reconstruction (iFace, clUGKS.c:134-195) in precision T ---------------
 __device__ __forceinline__ float rcp_T(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// WENO5 slopes of a (g, h) stencil: FP64 in weno5_slope_pair (ugks_device.hpp)
-__device__ __forceinline__ void weno5_pair(P2<double> s0, P2<double> s1, P2<double> s2, P2<double> s3, P2<double> s4,
-                                           double rdx, double &sgx, double &sgy) {
-    weno5_slope_pair(s0.x, s1.x, s2.x, s3.x, s4.x, s0.y, s1.y, s2.y, s3.y, s4.y, rdx, sgx, sgy);
-}
-__device__ __forceinline__ float weno5_f(float s0, float s1, float s2, float s3, float s4) {
+// WENO5 in FP32: the step from a stencil's middle cell to the face.  e_k =
+// 12 (eps + b_k) / sqrt(d_k) with the linear weights d = (0.1, 0.6, 0.3) riding
+// in the constants, and reciprocal estimates of the weights 1 / e_k^2.  Every
+// fused operation is written out: the results are rounded to FP32 again and
+// again, so the mixed plan keeps one order of operations whatever is built
+// around it.  (The FP64 form, weno5_q_pair in ugks_device.hpp, has fewer
+// operations, but would round every stored value of the mixed plan
+// differently.)  The passes specialised for WENO5 and the others (M = -1, and
+// the walls) fuse different terms of the middle candidate and of the sum.
+template <int M> __device__ __forceinline__ float weno5_f(float s0, float s1, float s2, float s3, float s4) {
     const float d1 = s1 - s0, d2 = s2 - s1, d3 = s3 - s2, d4 = s4 - s3;
-    const float u0 = d2 - d1, v0 = 3.f * d2 - d1;
+    const float u0 = d2 - d1, v0 = fmaf(3.f, d2, -d1);
     const float u1 = d3 - d2, v1 = d2 + d3;
-    const float u2 = d4 - d3, v2 = 3.f * d3 - d4;
+    const float u2 = d4 - d3, v2 = fmaf(3.f, d3, -d4);
     const float e0 = fmaf((float)kWA0 * u0, u0, fmaf((float)kWB0 * v0, v0, (float)kWE0));
     const float e1 = fmaf((float)kWA1 * u1, u1, fmaf((float)kWB1 * v1, v1, (float)kWE1));
     const float e2 = fmaf((float)kWA2 * u2, u2, fmaf((float)kWB2 * v2, v2, (float)kWE2));
     const float a0 = rcp_T(e0 * e0), a1 = rcp_T(e1 * e1), a2 = rcp_T(e2 * e2);
-    const float c0 = (-1.f / 3.f) * d1 + (5.f / 6.f) * d2;
-    const float c1 = (1.f / 6.f) * d2 + (1.f / 3.f) * d3;
-    const float c2 = (2.f / 3.f) * d3 - (1.f / 6.f) * d4;
-    return (a0 * c0 + a1 * c1 + a2 * c2) * rcp_T((a0 + a1) + a2);
-}
-__device__ __forceinline__ void weno5_pair(P2<float> s0, P2<float> s1, P2<float> s2, P2<float> s3, P2<float> s4,
-                                           float rdx, float &sgx, float &sgy) {
-    sgx = weno5_f(s0.x, s1.x, s2.x, s3.x, s4.x) * rdx;
-    sgy = weno5_f(s0.y, s1.y, s2.y, s3.y, s4.y) * rdx;
+    const float c0 = fmaf(5.f / 6.f, d2, -((1.f / 3.f) * d1));
+    const float c1 = M == 1 ? fmaf(1.f / 6.f, d2, (1.f / 3.f) * d3) : fmaf(1.f / 3.f, d3, (1.f / 6.f) * d2);
+    const float c2 = fmaf(2.f / 3.f, d3, -((1.f / 6.f) * d4));
+    const float n01 = M == 1 ? fmaf(a0, c0, a1 * c1) : fmaf(a1, c1, a0 * c0);
+    return fmaf(a2, c2, n01) * rcp_T((a0 + a1) + a2);
 }
 template <typename T> __device__ __forceinline__ T vanleer_T(T s1, T s2) {
     T a1 = s1 < T(0) ? -s1 : s1, a2 = s2 < T(0) ? -s2 : s2;
@@ -262,13 +262,19 @@ template <typename T> __device__ __forceinline__ void stream_store(__attribute__
     __builtin_nontemporal_store(x, p);
 }
 
+// element v of a wavefront-uniform row: the row stays a scalar base and the lane adds a 32-bit byte offset
+template <typename T> __device__ __forceinline__ AS1 V2<T> *vslot(AS1 V2<T> *row, int v) {
+    return (AS1 V2<T> *)((AS1 char *)row + (unsigned)v * (unsigned)sizeof(V2<T>));
+}
 // velocity table reads through global (not generic) pointers: they count only
 // against the vector-memory counter, so waiting for them does not also wait on LDS
 __device__ __forceinline__ d2 quad_at(const Consts &C, int v) {
-    const V2<double> x = ((const AS1 V2<double> *)C.quad)[v];
+    const V2<double> x = *vslot<double>((AS1 V2<double> *)C.quad, v);
     return d2{x.x, x.y};
 }
-__device__ __forceinline__ double weight_at(const Consts &C, int v) { return ((const AS1 double *)C.weight)[v]; }
+__device__ __forceinline__ double weight_at(const Consts &C, int v) {
+    return *(const AS1 double *)((const AS1 char *)C.weight + (unsigned)v * 8u);
+}
 // a wavefront-uniform double held in scalar registers (keeps per-face
 // constants out of VGPRs, so they are neither spilled nor recomputed in loops)
 __device__ __forceinline__ double uniform_d(double x) {
@@ -278,7 +284,8 @@ __device__ __forceinline__ double uniform_d(double x) {
 }
 // the reciprocals go through an empty asm so the compiler cannot turn the
 // per-lane select of two of them back into a division inside the velocity loop
-__device__ __forceinline__ void uniform_geo(FaceGeo &g) {
+template <typename T, int M> __device__ __forceinline__ void uniform_geo(FaceGeo &g) {
+    if constexpr (sizeof(T) == 8 && M == 1) return;       // the FP64 WENO5 needs no distance in the velocity loop
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         g.dist[k] = uniform_d(g.dist[k]);
@@ -301,8 +308,8 @@ template <typename T> __device__ __forceinline__ T geo_pick(const double (&d)[2]
     if constexpr (sizeof(T) == 4) return delta ? f[1] : f[0];
     else return delta ? d[1] : d[0];
 }
-template <typename T> __device__ __forceinline__ P2<T> sld(const Stencil<T> &st, unsigned rel, unsigned vb) {
-    const V2<T> x = *(const AS1 V2<T> *)(st.base + (rel * st.sb + vb));
+template <typename T> __device__ __forceinline__ P2<T> sld(const Stencil<T> &st, unsigned off) {
+    const V2<T> x = *(const AS1 V2<T> *)(st.base + off);
     return P2<T>{x.x, x.y};
 }
 
@@ -312,33 +319,39 @@ template <typename T> __device__ __forceinline__ P2<T> sld(const Stencil<T> &st,
 template <typename T> struct StenVals { P2<T> s0, s1, s2, s3, s4; };
 template <typename T, int M = -1>
 __device__ __forceinline__ void stencil_load(const Consts &C, const Stencil<T> &st, int v, int delta, StenVals<T> &x) {
-    const unsigned vb = (unsigned)v * (unsigned)sizeof(P2<T>);
+    // the lane's first stencil cell and its step to the next (both mod 2^32; every sum stays in the span)
+    const unsigned far = (method_of<M>(C) == 1 ? 5u : 3u) * st.sb;
+    unsigned off = (unsigned)v * (unsigned)sizeof(P2<T>) + (delta ? 0u : far);
+    const unsigned s = delta ? st.sb : 0u - st.sb;
+    x.s0 = sld<T>(st, off);
+    x.s1 = sld<T>(st, off += s);
+    x.s2 = sld<T>(st, off += s);
     if (method_of<M>(C) == 1) {
-        x.s0 = sld<T>(st, delta ? 0 : 5, vb);
-        x.s1 = sld<T>(st, delta ? 1 : 4, vb);
-        x.s2 = sld<T>(st, delta ? 2 : 3, vb);
-        x.s3 = sld<T>(st, delta ? 3 : 2, vb);
-        x.s4 = sld<T>(st, delta ? 4 : 1, vb);
+        x.s3 = sld<T>(st, off += s);
+        x.s4 = sld<T>(st, off += s);
     } else {
-        x.s0 = sld<T>(st, delta ? 0 : 3, vb);
-        x.s1 = sld<T>(st, delta ? 1 : 2, vb);
-        x.s2 = sld<T>(st, delta ? 2 : 1, vb);
         x.s3 = x.s4 = x.s2;
     }
 }
 
-// reconstructed face value and slope (iFace) from the stencil values; fl /
-// fr, the cells below / above the face, on request
+// The reconstructed face value (iFace) from the stencil values, and the slope
+// in units of slope_unit: the FP64 WENO5 gives six times the step from the
+// upwind cell's centre to the face, the others the slope itself.
+template <typename T> constexpr bool kUndivided = sizeof(T) == 8;
 template <typename T, int M = -1>
-__device__ __forceinline__ void reconstruct_from(const Consts &C, const FaceGeo &g, int delta, const StenVals<T> &x,
-                                                 P2<T> &ff, P2<T> &sg, P2<T> *fl = nullptr, P2<T> *fr = nullptr) {
+__device__ __forceinline__ void reconstruct_from(const Consts &C, const FaceGeo &g, int delta, const StenVals<T> &x, P2<T> &ff, P2<T> &sg) {
     if (method_of<M>(C) == 1) {
-        const T dist = geo_pick<T>(g.dist, g.fdist, delta), rdx = geo_pick<T>(g.rdist, g.frdist, delta);
-        weno5_pair(x.s0, x.s1, x.s2, x.s3, x.s4, rdx, sg.x, sg.y);
-        ff.x = x.s2.x + sg.x * dist;
-        ff.y = x.s2.y + sg.y * dist;
-        if (fl) *fl = P2<T>{delta ? x.s2.x : x.s3.x, delta ? x.s2.y : x.s3.y};
-        if (fr) *fr = P2<T>{delta ? x.s3.x : x.s2.x, delta ? x.s3.y : x.s2.y};
+        if constexpr (kUndivided<T>) {
+            weno5_q_pair(x.s0.x, x.s1.x, x.s2.x, x.s3.x, x.s4.x, x.s0.y, x.s1.y, x.s2.y, x.s3.y, x.s4.y, sg.x, sg.y);
+            ff.x = x.s2.x + sg.x * (1.0 / 6.0);
+            ff.y = x.s2.y + sg.y * (1.0 / 6.0);
+        } else {
+            const T dist = geo_pick<T>(g.dist, g.fdist, delta), rdx = geo_pick<T>(g.rdist, g.frdist, delta);
+            sg.x = weno5_f<M>(x.s0.x, x.s1.x, x.s2.x, x.s3.x, x.s4.x) * rdx;
+            sg.y = weno5_f<M>(x.s0.y, x.s1.y, x.s2.y, x.s3.y, x.s4.y) * rdx;
+            ff.x = fmaf(sg.x, dist, x.s2.x);
+            ff.y = fmaf(sg.y, dist, x.s2.y);
+        }
     } else {
         const T dist = geo_pick<T>(g.dist, g.fdist, delta);
         if (method_of<M>(C) == 0) {
@@ -352,17 +365,18 @@ __device__ __forceinline__ void reconstruct_from(const Consts &C, const FaceGeo 
         }
         ff.x = x.s1.x + sg.x * dist;
         ff.y = x.s1.y + sg.y * dist;
-        if (fl) *fl = P2<T>{delta ? x.s1.x : x.s2.x, delta ? x.s1.y : x.s2.y};
-        if (fr) *fr = P2<T>{delta ? x.s2.x : x.s1.x, delta ? x.s2.y : x.s1.y};
     }
+}
+template <typename T, int M> __device__ __forceinline__ double slope_unit(const Consts &C, const FaceGeo &g, int delta) {
+    return kUndivided<T> && method_of<M>(C) == 1 ? (1.0 / 6.0) * (delta ? g.rdist[1] : g.rdist[0]) : 1.0;
 }
 
 template <typename T>
 __device__ __forceinline__ void reconstruct(const Consts &C, const Stencil<T> &st, const FaceGeo &g, int v, int delta,
-                                            P2<T> &ff, P2<T> &sg, P2<T> *fl = nullptr, P2<T> *fr = nullptr) {
+                                            P2<T> &ff, P2<T> &sg) {
     StenVals<T> x;
     stencil_load<T>(C, st, v, delta, x);
-    reconstruct_from<T>(C, g, delta, x, ff, sg, fl, fr);
+    reconstruct_from<T>(C, g, delta, x, ff, sg);
 }
 
 #define AS3 __attribute__((address_space(3)))
@@ -421,6 +435,16 @@ __device__ __forceinline__ void stencil_read(const Consts &C, const AS3 char *lb
     }
 }
 
+// to_local with its fused operations written out (the mixed plan keeps one order of operations)
+__device__ __forceinline__ d2 to_face(d2 m, d2 n) { return d2{fma(m.y, n.y, m.x * n.x), fma(m.y, n.x, -(m.x * n.y))}; }
+
+// Waits around the staging buffer, written out: the compiler's own tracking of
+// loads into LDS loses them where a loop it has peeled joins its header (the
+// buffer was then read before the loads had landed).  The memory clobbers
+// keep its LDS reads between the two.
+__device__ __forceinline__ void stencil_landed() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ void stencil_consumed() { __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // Velocity loop of a wavefront-per-face pass, v = lane, lane + 64, ...: the
 // body gets the global velocity e, its weight w, the face-frame velocity uv,
 // the upwind choice and the stencil.  The stencil of the next velocity is
@@ -439,7 +463,8 @@ __device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stenci
     for (int v = lane; v < C.NV; v += 64) {
         const d2 ec = e;
         const double wc = w;
-        const d2 uv = d2{ec.x * n.x + ec.y * n.y, ec.x * (-n.y) + ec.y * n.x};     // face_velocity
+        const d2 uv = to_face(ec, n);
+
         const int delta = upwind(uv.x);
         StenVals<T> cur;
         // the next velocity's table entries, or this one's again on the last
@@ -448,9 +473,9 @@ __device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stenci
         // in flight when the wavefront leaves the loop.
         const int vn = v + 64 < C.NV ? v + 64 : v;
         if constexpr (LDS) {
+            stencil_landed();
             stencil_read<T, M>(C, lb, lane, delta, cur);
-            // the reads have returned before the next loads overwrite the buffer
-            __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+            stencil_consumed();   // the reads have returned before the next loads overwrite the buffer
             e = quad_at(C, vn);
             w = weight_at(C, vn);
             if (v + 64 < C.NV) {
@@ -466,29 +491,31 @@ __device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stenci
     }
 }
 
-// the cells below (rel R-1) and above (rel R, the owner) the face
-template <typename T>
-__device__ __forceinline__ void face_cells(const Consts &C, const Stencil<T> &st, int v, P2<T> &fl, P2<T> &fr) {
-    const unsigned vb = (unsigned)v * (unsigned)sizeof(P2<T>);
-    const unsigned R = C.method == 1 ? 3 : 2;
-    fl = sld<T>(st, R - 1, vb);
-    fr = sld<T>(st, R, vb);
-}
-
 // ============================================================ face passes ==
 // Faces are numbered so that neighbouring ids share stencil cells: S faces
 // column by column (j fastest), W faces row by row (i fastest).
 // Per interior face: (A) one wavefront reconstructs f at the face for every
 // velocity and sums the raw face moments (the conserved moments of
-// getFaceCons, the third-order ones the face heat flux of calcFaceQ needs,
-// clUGKS.c:522-585), the left/right cell moments (getAL/getAR) and the owner
-// cell's heat flux (calcQ); (S) one thread turns those sums into the face
-// state (getPLR, initMacroFlux, calcFaceQ); (C) one wavefront rebuilds the
-// face values and forms the per-velocity flux (distFlux) and the macro flux
-// (macroFlux).  Face ids: per block, S faces then W faces (walls excluded).
-constexpr int kNS = 15;   // face sums: 13 raw moments of the face values, the owner's heat flux
-constexpr int kFS = 16;   // face sums per face (padded)
-constexpr int kFT = 32;   // face state per face
+// getFaceCons and the third-order ones the face heat flux of calcFaceQ needs,
+// clUGKS.c:522-585) in the global frame; (S) one thread turns those sums, the
+// cell moments (getAL/getAR) and the geometry into the face state (getPLR,
+// initMacroFlux, calcFaceQ); (C) one wavefront rebuilds the face values and
+// forms the per-velocity flux (distFlux) and the macro flux (macroFlux).
+// Face ids: per block, S faces then W faces (walls excluded).
+//
+// The FP64 plan's face sums, with e the velocity and E = |e|^2: 0 g, 1-2 e g,
+// 3 ex^2 g, 4 ey^2 g, 5 ex ey g, 6-7 E e g, 8 h, 9-10 e h.  The heat flux only
+// needs the contracted third moment, which rotates as a vector, so no velocity
+// is rotated in the loop and 11 sums do.  (With the shorter WENO5 and the cell's
+// heat flux left to the update the pass went 0.85 -> 0.75 ms on 2 x 2 blocks of
+// 128^2 cells with 33^2 velocities.)  The mixed plan's sums are the face
+// frame's, 0 g, 1 u g, 2 w g, 3 u^2 g, 4 w^2 g, 5 u w g, 6 u^3 g, 7 w^3 g,
+// 8 u w^2 g, 9 u^2 w g, 10 h, 11 u h, 12 w h: its f is rounded to FP32 every
+// step, where a last-bit difference in these sums would now and then turn a
+// stored value by one unit, so their order of operations is kept.
+template <typename T> constexpr int kFS = sizeof(T) == 8 ? 12 : 13;   // face sums per face
+inline int kFSof(int precision) { return precision == UGKS_FP64 ? kFS<double> : kFS<float>; }
+constexpr int kFT = 32;                                               // face state per face
 
 struct FaceLoc { int face, mi, mj, gi, gj; };
 __device__ __forceinline__ FaceLoc face_loc(const FBlock &B, long long loc) {
@@ -601,48 +628,75 @@ __global__ void __launch_bounds__(64 * FW) k_faceA(const FBlock *__restrict__ bl
     const FaceRec R = recs[sid];
     const FBlock &B = blocks[R.b];
     const Consts &C = B.c;
-    const FaceLoc L{R.face, R.gi - C.G, R.gj - C.G, R.gi, R.gj};
     FaceGeo g = face_geo_of(R, C);
-    uniform_geo(g);
+    uniform_geo<T, M>(g);
     const Stencil<T> stn = stencil<T, M>(C, B.f, g);
-    const d2 n = B.normal[g.own * 2 + L.face];
-    const bool wantQ = (L.face == SOUTH) && (L.mj < C.nj);
-    const d4 cm = wantQ ? B.macro[(size_t)L.mi * C.nj + L.mj] : mk4(0, 0, 0, 1);
-    const double rK = 1.0 / C.K;
-    double a[kFS];            // kNS sums and one pad, so the reduction folds 16
+    const d2 n = B.normal[g.own * 2 + R.face];
+    constexpr int NR = sizeof(T) == 8 ? 3 : 4;                // sums per row of the wavefront
+    double a[4 * NR];
 #pragma unroll
-    for (int q = 0; q < kFS; q++) a[q] = 0.0;
-    face_velocity_loop<T, M, false>(C, stn, n, lane, nullptr, [&](int v, d2 e, double, d2 uv, int delta, const StenVals<T> &sv) __attribute__((always_inline)) {
-        P2<T> ff, sg, fl, fr;
-        reconstruct_from<T, M>(C, g, delta, sv, ff, sg, &fl, &fr);
-        const double u = uv.x, w = uv.y, gx = (double)ff.x, hx = (double)ff.y;
-        const double ug = u * gx, wg = w * gx, uug = u * ug, wwg = w * wg;
-        a[0] += gx; a[1] += ug; a[2] += wg;
-        a[3] += uug; a[4] += wwg; a[5] += u * wg;
-        a[6] += u * uug; a[7] += w * wwg; a[8] += u * wwg; a[9] += w * uug;
-        a[10] += hx; a[11] += u * hx; a[12] += w * hx;
-        if (wantQ) {
-            const double x = (double)fr.x, y = (double)fr.y;
-            const double cx = e.x - cm.s1, cy = e.y - cm.s2, t = (cx * cx + cy * cy) * x + y * rK;
-            a[13] += 0.5 * (cx * t);
-            a[14] += 0.5 * (cy * t);
+    for (int q = 0; q < 4 * NR; q++) a[q] = 0.0;
+    if (lane < C.NV) {
+        d2 e = quad_at(C, lane);
+        for (int v = lane; v < C.NV; v += 64) {
+            const d2 ec = e;
+            const double un = fma(ec.y, n.y, ec.x * n.x);
+            const int delta = upwind(un);
+            // the next velocity, or this one again on the last round: no branch
+            e = quad_at(C, v + 64 < C.NV ? v + 64 : v);
+            StenVals<T> sv;
+            stencil_load<T, M>(C, stn, v, delta, sv);
+            P2<T> ff, sg;
+            reconstruct_from<T, M>(C, g, delta, sv, ff, sg);
+            const double gg = (double)ff.x, hh = (double)ff.y;
+            if constexpr (sizeof(T) == 8) {
+                const double x = ec.x, y = ec.y, xg = x * gg, yg = y * gg, Eg = fma(x, xg, y * yg);
+                a[0] += gg; a[1] += xg; a[2] += yg;
+                a[3] = fma(x, xg, a[3]); a[4] = fma(y, yg, a[4]); a[5] = fma(x, yg, a[5]);
+                a[6] = fma(x, Eg, a[6]); a[7] = fma(y, Eg, a[7]);
+                a[8] += hh; a[9] = fma(x, hh, a[9]); a[10] = fma(y, hh, a[10]);
+            } else {
+                const double u = un, w = fma(ec.y, n.x, -(ec.x * n.y));
+                const double ug = u * gg, wg = w * gg, uug = u * ug, wwg = w * wg;
+                a[0] += gg; a[1] += ug; a[2] += wg;
+                a[3] += uug; a[4] += wwg; a[5] += u * wg;
+                a[6] += u * uug; a[7] += w * wwg; a[8] += u * wwg; a[9] += w * uug;
+                a[10] += hh; a[11] += u * hh; a[12] += w * hh;
+            }
         }
-    });
-    // row r of the wavefront gets the totals of sums 4r .. 4r+3; its first
-    // lane stores them (the pad, sum 15, is zero)
-    double t[4];
-    wave_sum16_rows(a, t);
-    if ((lane & 15) == 0) {
-        d2 *o = (d2 *)(fsum + sid * kFS + 4 * (lane >> 4));
-        o[0] = mk2(t[0], t[1]);
-        o[1] = mk2(t[2], t[3]);
-        if (wantQ && lane == 48) B.Q[(size_t)L.mi * C.nj + L.mj] = mk2(t[1], t[2]);
     }
+    // row r of the wavefront gets the totals of sums NR r .. NR r + NR - 1; its first lane stores them
+    double t[NR];
+    wave_sum_rows<NR>(a, t);
+    if ((lane & 15) == 0) {
+        const int k = NR * (lane >> 4);
+        double *o = fsum + sid * kFS<T> + k;
+#pragma unroll
+        for (int q = 0; q < NR; q++)
+            if (k + q < kFS<T>) o[q] = t[q];
+    }
+}
+
+// conserved moments and heat flux (about (U, V), face frame) from the FP64 plan's face sums
+__device__ __forceinline__ d4 face_moments(const double *S, d2 n) {
+    const d2 m = to_local(mk2(S[1], S[2]), n);
+    return mk4(S[0], m.x, m.y, 0.5 * ((S[3] + S[4]) + S[8]));
+}
+__device__ __forceinline__ d2 face_heat(const double *S, d2 n, double U, double V, double K) {
+    const double E = S[3] + S[4], nxy = n.x * n.y, c = U * U + V * V;
+    const d2 m1 = to_local(mk2(S[1], S[2]), n), m3 = to_local(mk2(S[6], S[7]), n), mh = to_local(mk2(S[9], S[10]), n);
+    const double uu = n.x * n.x * S[3] + 2.0 * nxy * S[5] + n.y * n.y * S[4];
+    const double ww = n.y * n.y * S[3] - 2.0 * nxy * S[5] + n.x * n.x * S[4];
+    const double uw = nxy * (S[4] - S[3]) + (n.x * n.x - n.y * n.y) * S[5];
+    const double c2 = E - 2.0 * (U * m1.x + V * m1.y) + c * S[0];         // sum |c - (U, V)|^2 g
+    return mk2(0.5 * ((m3.x - 2.0 * (U * uu + V * uw) + c * m1.x - U * c2) + (mh.x - U * S[8]) / K),
+               0.5 * ((m3.y - 2.0 * (U * uw + V * ww) + c * m1.y - V * c2) + (mh.y - V * S[8]) / K));
 }
 
 // face state: primary variables, slopes, time slope, time integrals, the
 // equilibrium part of the macro flux and the face heat flux (from the raw
 // moments about the face velocity) -- getPLR, initMacroFlux, calcFaceQ
+template <typename T>
 __global__ void __launch_bounds__(kT) k_faceS(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
                                               long long nfaces, const double *__restrict__ fsum,
                                               double *__restrict__ fstate, const DtState *__restrict__ ds) {
@@ -654,12 +708,14 @@ __global__ void __launch_bounds__(kT) k_faceS(const FBlock *__restrict__ blocks,
     const FaceLoc L{R.face, R.gi - C.G, R.gj - C.G, R.gi, R.gj};
     const size_t own = (size_t)L.gi * C.NJ + L.gj;
     const long long step = L.face == SOUTH ? 1 : C.NJ;
-    const double *S = fsum + fid * kFS;
-    const d4 W = mk4(S[0], S[1], S[2], 0.5 * ((S[3] + S[4]) + S[10]));
+    const double *S = fsum + fid * kFS<T>;
+    const d2 n = B.normal[own * 2 + L.face];
+    d4 W;
+    if constexpr (sizeof(T) == 8) W = face_moments(S, n);
+    else W = mk4(S[0], S[1], S[2], 0.5 * ((S[3] + S[4]) + S[10]));
     // getAL / getAR: the moments of the cells below and above the face in face coordinates
-    const d2 nf = B.normal[own * 2 + L.face];
     const d4 ML = B.cmom[(long long)own - step], MR = B.cmom[own];
-    const d2 uL = to_local(mk2(ML.s1, ML.s2), nf), uR = to_local(mk2(MR.s1, MR.s2), nf);
+    const d2 uL = to_face(mk2(ML.s1, ML.s2), n), uR = to_face(mk2(MR.s1, MR.s2), n);
     const d4 WL = mk4(ML.s0, uL.x, uL.y, ML.s3), WR = mk4(MR.s0, uR.x, uR.y, MR.s3);
     const d4 prim = to_primary(C, W);
     // |midside - centre| of the cells below (upwind choice 1) and above (0) the face
@@ -675,13 +731,18 @@ __global__ void __launch_bounds__(kT) k_faceS(const FBlock *__restrict__ blocks,
                              mt.m2 * moment_au(aT, m.Mu, m.Mv, m.Mxi, 1, 0));
     // face heat flux 1/2 sum (c-U)(|c-U|^2 g + h/K) from the raw moments
     const double U = prim.s1, V = prim.s2;
-    const double qx = 0.5 * ((S[6] - 3.0 * U * S[3] + 3.0 * U * U * S[1] - U * U * U * S[0]) +
-                             (S[8] - 2.0 * V * S[5] + V * V * S[1] - U * S[4] + 2.0 * U * V * S[2] - U * V * V * S[0]) +
-                             (S[11] - U * S[10]) / C.K);
-    const double qy = 0.5 * ((S[7] - 3.0 * V * S[4] + 3.0 * V * V * S[2] - V * V * V * S[0]) +
-                             (S[9] - 2.0 * U * S[5] + U * U * S[2] - V * S[3] + 2.0 * U * V * S[1] - V * U * U * S[0]) +
-                             (S[12] - V * S[10]) / C.K);
-    const d2 n = B.normal[own * 2 + L.face];
+    double qx, qy;
+    if constexpr (sizeof(T) == 8) {
+        const d2 q = face_heat(S, n, U, V, C.K);
+        qx = q.x; qy = q.y;
+    } else {
+        qx = 0.5 * ((S[6] - 3.0 * U * S[3] + 3.0 * U * U * S[1] - U * U * U * S[0]) +
+                    (S[8] - 2.0 * V * S[5] + V * V * S[1] - U * S[4] + 2.0 * U * V * S[2] - U * V * V * S[0]) +
+                    (S[11] - U * S[10]) / C.K);
+        qy = 0.5 * ((S[7] - 3.0 * V * S[4] + 3.0 * V * V * S[2] - V * V * V * S[0]) +
+                    (S[9] - 2.0 * U * S[5] + U * U * S[2] - V * S[3] + 2.0 * U * V * S[1] - V * U * U * S[0]) +
+                    (S[12] - V * S[10]) / C.K);
+    }
     // The per-velocity flux (distFlux) with its per-face factors folded, so the
     // flux pass evaluates, for P_a = a0 + a1 u + a2 w + a3 |u|^2 / 2,
     //   Q_side = m1 (P_side + hk a3 / 2)        (side = L or R, by the upwind choice)
@@ -709,100 +770,214 @@ __global__ void __launch_bounds__(kT) k_faceS(const FBlock *__restrict__ blocks,
     o[28] = Lf; o[29] = n.x; o[30] = n.y; o[31] = 0.0;
 }
 
+// The flux pass's per-face tables on a tensor velocity grid whose face normal
+// lies along an axis: the factors of the per-velocity flux that depend on the
+// normal velocity alone (N, 5 pairs per grid value) or on the tangential one
+// alone (T, 3 pairs).  A pair is one 16-byte LDS read; an odd number of pairs
+// per entry spreads consecutive entries over all banks.  The FP64 plan folds
+// everything that factorises; the mixed one keeps the order of operations of
+// the general loop (its flux is rounded to FP32, see the face sums).
+constexpr int kTabN = 5 * 16, kTabT = 3 * 16;
+constexpr int kTabBytes = kTabN + kTabT;          // LDS bytes per wavefront and grid value of the longer axis
+__device__ __forceinline__ V2<double> lpair(const AS3 char *p) { return *(const AS3 V2<double> *)p; }
+__device__ __forceinline__ void put_pair(AS3 char *p, double x, double y) { *(AS3 V2<double> *)p = V2<double>{x, y}; }
+
+// the face's folded flux constants (k_faceS)
+struct FluxState {
+    double U, V, lam, hk;
+    d4 QL, QR, QT;
+    double DL, DR, DT, m3, m4;
+    d2 SQ;
+    double rl;
+};
+__device__ __forceinline__ FluxState flux_state(const double *sv) {
+    return FluxState{sv[0], sv[1], sv[2], sv[3], mk4(sv[4], sv[5], sv[6], sv[7]), mk4(sv[8], sv[9], sv[10], sv[11]),
+                     mk4(sv[12], sv[13], sv[14], sv[15]), sv[16], sv[17], sv[18], sv[19], sv[20], mk2(sv[21], sv[22]), sv[23]};
+}
+// table entry of normal velocity u / tangential velocity w, c the velocity
+// less the face's mean, E = exp(-lam c^2) (unit: slope_unit of both upwind choices)
+template <typename T>
+__device__ __forceinline__ void put_normal(AS3 char *p, const FluxState &s, d2 unit, double u, double c, double E) {
+    const bool up = upwind(u);
+    const double q0 = up ? s.QL.s0 : s.QR.s0, q1 = up ? s.QL.s1 : s.QR.s1, q2 = up ? s.QL.s2 : s.QR.s2, q3 = up ? s.QL.s3 : s.QR.s3;
+    const double D = fma(u, up ? s.DL : s.DR, s.DT);
+    if constexpr (sizeof(T) == 8) {
+        const double uu = u * u;
+        put_pair(p, fma(u, q0 + q1 * u + q3 * uu, s.QT.s0 + s.QT.s1 * u + s.QT.s3 * uu), fma(u, q2, s.QT.s2));
+        put_pair(p + 16, fma(u, q3, s.QT.s3), c * s.SQ.x);
+        put_pair(p + 32, fma(2.0 * s.lam * c, c, -4.0), D);
+        put_pair(p + 48, s.rl * E, s.m4 * u * (up ? unit.y : unit.x));
+        put_pair(p + 64, u, uu);
+    } else {
+        put_pair(p, fma(q1, u, q0), q2);
+        put_pair(p + 16, q3, fma(s.QT.s1, u, s.QT.s0));
+        put_pair(p + 32, D, s.m4 * u);
+        put_pair(p + 48, E, 0.0);
+        put_pair(p + 64, u, c);
+    }
+}
+template <typename T>
+__device__ __forceinline__ void put_tangential(AS3 char *p, const FluxState &s, double w, double c, double E) {
+    put_pair(p, w, w * w);
+    if constexpr (sizeof(T) == 8) put_pair(p + 16, c * s.SQ.y, 2.0 * s.lam * c * c);
+    else put_pair(p + 16, c * s.SQ.y, c * c);
+    put_pair(p + 32, E, 0.0);
+}
+
 // minimum wavefronts per SIMD asked of the flux pass: the FP32 variants with a
 // fixed reconstruction run six (80 VGPRs; WENO5 spills 4 registers there and
 // is still faster than at five); the others are left to the compiler
 template <typename T, int M> constexpr int kFaceCWaves = (sizeof(T) == 4 && M >= 0) ? 6 : 1;
 // the FP64 flux stores one iteration late (the FP32 variant would spill more at six waves)
 template <typename T> constexpr bool kDeferStore = sizeof(T) == 8;
-template <typename T, int FW, int M>
-__global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kFaceCWaves<T, M>))) k_faceC(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
-                                                   long long nfaces, const double *__restrict__ fstate) {
-    __shared__ double tab[FW][128];
-    __shared__ __attribute__((aligned(16))) char sbuf[FW][kStenLds<T>];
-    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const long long fid = xcd_remap(blockIdx.x, gridDim.x) * FW + wv;
-    if (fid >= nfaces) return;
-    const int lane = threadIdx.x & 63;
-    const FaceRec R = recs[fid];
-    const FBlock &B = blocks[R.b];
-    const Consts &C = B.c;
-    const FaceLoc L{R.face, R.gi - C.G, R.gj - C.G, R.gi, R.gj};
-    FaceGeo g = face_geo_of(R, C);
-    uniform_geo(g);
-    const Stencil<T> stn = stencil<T, M>(C, B.f, g);
-    // the face's folded flux constants (k_faceS)
-    const double *sv = fstate + fid * kFT;
-    const double U = sv[0], V = sv[1], lam = sv[2], hk = sv[3];
-    const d4 QL = mk4(sv[4], sv[5], sv[6], sv[7]), QR = mk4(sv[8], sv[9], sv[10], sv[11]);
-    const d4 QT = mk4(sv[12], sv[13], sv[14], sv[15]);
-    const double DL = sv[16], DR = sv[17], DT = sv[18], m3 = sv[19], m4 = sv[20];
-    const d2 SQ = mk2(sv[21], sv[22]);
-    const double rl = sv[23], Lf = sv[28];
-    const d2 n = mk2(sv[29], sv[30]);
-    // separable Maxwellian on a tensor grid with an axis-aligned normal:
-    // exp(-lam |uv - (U,V)|^2) = Ei[v / nvt] * Ej[v % nvt], one table pair per wave in LDS
-    const bool sep = C.nut > 0 && (n.x == 0.0 || n.y == 0.0);
-    double *Ei = tab[wv], *Ej = tab[wv] + 64;
-    if (sep) {
-        const bool wtype = (n.y == 0.0);
-        if (lane < C.nut) {
-            const double a = wtype ? n.x * C.qu[lane] : -n.y * C.qu[lane], c = wtype ? U : V;
-            Ei[lane] = exp(-lam * ((a - c) * (a - c)));
+
+// Velocity loop of one face through the tables.  WT: the normal runs along u
+// (the slow velocity index), else along v (the fast one).  mf collects the
+// macro flux sums.
+template <typename T, int M, bool WT>
+__device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, int lane,
+                                                 AS3 char *sb, AS3 char *tabN, AS3 char *tabT, AS1 V2<T> *fout, double (&mf)[4]) {
+    constexpr bool LDS = kStenViaLds<T>;
+    const int NV = C.NV, nvt = __builtin_amdgcn_readfirstlane(C.nvt);
+    if (lane >= NV) return;
+    // LDS addresses of this lane's slow and fast table entries, advanced without division
+    constexpr int ss = WT ? kTabN : kTabT, sf = WT ? kTabT : kTabN;
+    const int iu0 = lane / nvt, jv0 = lane - iu0 * nvt, diu = 64 / nvt, djv = 64 - diu * nvt;
+    AS3 char *ps = (WT ? tabN : tabT) + iu0 * ss, *pf = (WT ? tabT : tabN) + jv0 * sf;
+    AS3 char *const pend_f = (WT ? tabT : tabN) + nvt * sf;
+    double w = weight_at(C, lane);
+    unsigned vb = (unsigned)lane * (unsigned)sizeof(P2<T>);
+    if constexpr (LDS) stencil_dma<T, M>(C, stn, vb, sb);
+    V2<T> pend = V2<T>{T(0), T(0)};
+    int last = -1;
+    for (int v = lane; v < NV; v += 64) {
+        const AS3 char *pn = WT ? ps : pf, *pt = WT ? pf : ps;
+        const V2<double> n4 = lpair(pn + 64);
+        const double ux = n4.x;
+        const int delta = upwind(ux);
+        const double wc = w;
+        StenVals<T> cur;
+        const int vn = v + 64 < NV ? v + 64 : v;
+        if constexpr (LDS) {
+            stencil_landed();
+            stencil_read<T, M>(C, sb, lane, delta, cur);
+            stencil_consumed();   // the reads have returned before the next loads overwrite the buffer
+            w = weight_at(C, vn);
+            if (v + 64 < NV) {
+                vb += 64u * (unsigned)sizeof(P2<T>);
+                stencil_dma<T, M>(C, stn, vb, sb);
+            }
+        } else {
+            w = weight_at(C, vn);
+            stencil_load<T, M>(C, stn, v, delta, cur);
         }
-        if (lane < C.nvt) {
-            const double a = wtype ? n.x * C.qv[lane] : n.y * C.qv[lane], c = wtype ? V : U;
-            Ej[lane] = exp(-lam * ((a - c) * (a - c)));
+        if constexpr (kDeferStore<T>) {
+            if (v >= 64) stream_store<T>(vslot<T>(fout, v - 64), pend);
+            last = v;
         }
+        P2<T> ff, sg;
+        reconstruct_from<T, M>(C, g, delta, cur, ff, sg);
+        const V2<double> n0 = lpair(pn), n1 = lpair(pn + 16), n2 = lpair(pn + 32);
+        const V2<double> t0 = lpair(pt), t1 = lpair(pt + 16);
+        const double Ej = *(const AS3 double *)(pt + 32), uy = t0.x;
+        double rg, rh;
+        if constexpr (sizeof(T) == 8) {
+            const V2<double> n3 = lpair(pn + 48);
+            const double Bg = fma(n1.x, t0.y, fma(n0.y, uy, n0.x));
+            const double S = n1.y + t1.x, SP4 = S * (n2.x + t1.y), SP2 = fma(2.0, S, SP4);
+            const double f0 = wc * (n3.x * Ej), h0 = s.hk * f0;
+            const double tg = fma(s.m3, ff.x, -(n3.y * sg.x)), th = fma(s.m3, ff.y, -(n3.y * sg.y));
+            const double yg = fma(f0, SP4, tg), yh = fma(h0, SP2, th);      // the Shakhov and the non-equilibrium parts
+            rg = ux * fma(f0, Bg, yg);
+            rh = ux * fma(h0, Bg, fma(f0, n2.y, yh));
+            // macroFlux (clUGKS.c:607-661); mf[3] collects twice the energy flux here
+            const double X = ux * yg;
+            mf[0] += X;
+            mf[1] = fma(ux, X, mf[1]);
+            mf[2] = fma(uy, X, mf[2]);
+            mf[3] = fma(n4.y + t0.y, X, fma(ux, yh, mf[3]));
+        } else {
+            const double Ei = *(const AS3 double *)(pn + 48), cx = n4.y;
+            const double uu = fma(ux, ux, t0.y), c2 = fma(cx, cx, t1.y);
+            const double Qa = fma(n1.x, uu, fma(n0.y, uy, n0.x));
+            const double Bg = fma(ux, Qa, fma(s.QT.s3, uu, fma(s.QT.s2, uy, n1.y)));
+            const double S = fma(cx, s.SQ.x, t1.x), SP4 = S * fma(2.0 * s.lam, c2, -4.0), SP2 = fma(2.0, S, SP4);
+            const double f0 = wc * (s.rl * (Ei * Ej));
+            const double tg = fma(s.m3, (double)ff.x, -(n2.y * (double)sg.x)), th = fma(s.m3, (double)ff.y, -(n2.y * (double)sg.y));
+            rg = ux * fma(f0, Bg + SP4, tg);
+            rh = ux * fma(f0, fma(s.hk, Bg + SP2, n2.x), th);
+            const double X = ux * fma(SP4, f0, tg);
+            mf[0] += X;
+            mf[1] = fma(ux, X, mf[1]);
+            mf[2] = fma(uy, X, mf[2]);
+            mf[3] = fma(0.5, fma(uu, X, ux * fma(SP2, s.hk * f0, th)), mf[3]);
+        }
+        if constexpr (kDeferStore<T>) pend = V2<T>{(T)rg, (T)rh};
+        else stream_store<T>(vslot<T>(fout, v), V2<T>{(T)rg, (T)rh});
+        ps += diu * ss; pf += djv * sf;
+        if (pf >= pend_f) { pf -= nvt * sf; ps += ss; }
+    }
+    if (last >= 0) stream_store<T>(vslot<T>(fout, last), pend);
+    if constexpr (sizeof(T) == 8) mf[3] *= 0.5;
+}
+
+// Velocity loop of one face for any normal and velocity set: face-frame
+// velocities and polynomials formed per velocity.  On a tensor grid the FP64
+// plan's Maxwellian still factorises, in the global frame (its argument does
+// not depend on the frame): Ei[v / nvt] * Ej[v % nvt].
+template <typename T, int M>
+__device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, d2 n, int lane,
+                                                  AS3 char *sb, AS3 double *Ei, int nmax, AS1 V2<T> *fout, double (&mf)[4]) {
+    const bool tensor = sizeof(T) == 8 && C.nut > 0;
+    AS3 double *Ej = Ei + nmax;
+    if (tensor) {
+        const d2 Ug = to_global(mk2(s.U, s.V), n);
+        if (lane < C.nut) { const double c = C.qu[lane] - Ug.x; Ei[lane] = exp(-s.lam * (c * c)); }
+        if (lane < C.nvt) { const double c = C.qv[lane] - Ug.y; Ej[lane] = exp(-s.lam * (c * c)); }
     }
     // the tables are private to this wavefront: order its LDS writes before its reads
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    AS1 V2<T> *fout = (AS1 V2<T> *)(L.face == SOUTH ? B.fluxS : B.fluxW) + g.own * (size_t)C.NV;
-    const double lam2 = 2.0 * lam;
-    double mf[4] = {0.0, 0.0, 0.0, 0.0};
+    const double lam2 = 2.0 * s.lam, m4L = s.m4 * slope_unit<T, M>(C, g, 1), m4R = s.m4 * slope_unit<T, M>(C, g, 0);
     // tensor indices of v = lane + 64 k, advanced without integer division
     int iu = 0, jv = 0, diu = 0, djv = 0;
     // the grid width in a register: the flux stores could alias the block
     // record, so C.nvt would otherwise be loaded again in every iteration
     const int nvt = __builtin_amdgcn_readfirstlane(C.nvt);
-    if (sep) { iu = lane / nvt; jv = lane - iu * nvt; diu = 64 / nvt; djv = 64 - diu * nvt; }
+    if (tensor) { iu = lane / nvt; jv = lane - iu * nvt; diu = 64 / nvt; djv = 64 - diu * nvt; }
     // each velocity's flux is stored one iteration late, at the start of the
     // next, so the wait for the loads issued there does not also wait for it
     V2<T> pend = V2<T>{T(0), T(0)};
     int last = -1;
-    face_velocity_loop<T, M, kStenViaLds<T>>(C, stn, n, lane, (AS3 char *)sbuf[wv], [&](int v, d2, double wv, d2 uv, int delta, const StenVals<T> &stv) __attribute__((always_inline)) {
+    face_velocity_loop<T, M, kStenViaLds<T>>(C, stn, n, lane, sb, [&](int v, d2, double wv, d2 uv, int delta, const StenVals<T> &stv) __attribute__((always_inline)) {
         if constexpr (kDeferStore<T>) {
             if (v >= 64) stream_store<T>(fout + (v - 64), pend);
             last = v;
         }
         P2<T> ff, sg;
         reconstruct_from<T, M>(C, g, delta, stv, ff, sg);
-        const double ux = uv.x, uy = uv.y, cx = ux - U, cy = uy - V, c2 = cx * cx + cy * cy;
-        const double E = sep ? Ei[iu] * Ej[jv] : exp(-lam * c2);
-        if (sep) {
+        const double ux = uv.x, uy = uv.y, cx = ux - s.U, cy = uy - s.V, c2 = cx * cx + cy * cy;
+        const double E = tensor ? Ei[iu] * Ej[jv] : exp(-s.lam * c2);
+        if (tensor) {
             iu += diu; jv += djv;
             if (jv >= nvt) { jv -= nvt; iu++; }
         }
-        const double f0 = wv * (rl * E);                       // Lf f0 of g; hk f0 is h's
+        const double f0 = wv * (s.rl * E);                     // Lf f0 of g; hk f0 is h's
         const double uu = ux * ux + uy * uy;
-        double PL = QL.s0 + QL.s1 * ux + QL.s2 * uy + QL.s3 * uu, PR = QR.s0 + QR.s1 * ux + QR.s2 * uy + QR.s3 * uu;
+        double PL = s.QL.s0 + s.QL.s1 * ux + s.QL.s2 * uy + s.QL.s3 * uu, PR = s.QR.s0 + s.QR.s1 * ux + s.QR.s2 * uy + s.QR.s3 * uu;
         // FP32 storage: both sides' polynomials are evaluated and one is picked
         // per lane.  Left to itself the compiler picks the coefficients instead,
-        // which costs two moves per select (a select takes one scalar operand):
-        // 19 more VALU per velocity.  The FP64 variant keeps the compiler's
-        // form: with fewer VGPRs it runs four waves per SIMD, and measured
-        // slower there (1.43 -> 1.50 ms on 2x2 blocks of 128^2 cells, 33^2 velocities).
+        // which costs two moves per select (a select takes one scalar operand).
         if constexpr (sizeof(T) == 4) __asm__ volatile("" : "+v"(PL), "+v"(PR));
-        const double Qa = delta ? PL : PR, Da = delta ? DL : DR;
-        const double Bg = fma(ux, Qa, QT.s0 + QT.s1 * ux + QT.s2 * uy + QT.s3 * uu);
-        const double S = cx * SQ.x + cy * SQ.y, SP4 = S * fma(lam2, c2, -4.0), SP2 = fma(2.0, S, SP4);
+        const double Qa = delta ? PL : PR, Da = delta ? s.DL : s.DR;
+        const double Bg = fma(ux, Qa, s.QT.s0 + s.QT.s1 * ux + s.QT.s2 * uy + s.QT.s3 * uu);
+        const double S = cx * s.SQ.x + cy * s.SQ.y, SP4 = S * fma(lam2, c2, -4.0), SP2 = fma(2.0, S, SP4);
         const double fdg = (double)ff.x, fdh = (double)ff.y, slg = (double)sg.x, slh = (double)sg.y;
-        const double m4u = m4 * ux;
-        const double tg = m3 * fdg - m4u * slg, th = m3 * fdh - m4u * slh;
+        const double m4u = (delta ? m4L : m4R) * ux;
+        const double tg = s.m3 * fdg - m4u * slg, th = s.m3 * fdh - m4u * slh;
         const double rg = ux * fma(f0, Bg + SP4, tg);
-        const double rh = ux * fma(f0, fma(hk, Bg + SP2, fma(ux, Da, DT)), th);
+        const double rh = ux * fma(f0, fma(s.hk, Bg + SP2, fma(ux, Da, s.DT)), th);
         if constexpr (kDeferStore<T>) pend = V2<T>{(T)rg, (T)rh};
         else stream_store<T>(fout + v, V2<T>{(T)rg, (T)rh});
         // macroFlux (clUGKS.c:607-661): the Shakhov and the non-equilibrium parts
@@ -810,15 +985,73 @@ __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kF
         mf[0] += X;
         mf[1] += ux * X;
         mf[2] += uy * X;
-        mf[3] += 0.5 * (uu * X + ux * fma(SP2, hk * f0, th));
+        mf[3] += 0.5 * (uu * X + ux * fma(SP2, s.hk * f0, th));
     });
     if (last >= 0) stream_store<T>(fout + last, pend);
+}
+
+template <typename T, int FW, int M>
+__global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kFaceCWaves<T, M>))) k_faceC(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
+                                                   long long nfaces, const double *__restrict__ fstate, int nmax) {
+    // per wavefront: the stencil staging buffer, then the tables
+    extern __shared__ __attribute__((aligned(16))) char fc_lds[];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long fid = xcd_remap(blockIdx.x, gridDim.x) * FW + wv;
+    if (fid >= nfaces) return;
+    const int lane = threadIdx.x & 63;
+    AS3 char *sb = (AS3 char *)fc_lds + wv * (kStenLds<T> + kTabBytes * nmax), *tab = sb + kStenLds<T>;
+    const FaceRec R = recs[fid];
+    const FBlock &B = blocks[R.b];
+    const Consts &C = B.c;
+    FaceGeo g = face_geo_of(R, C);
+    uniform_geo<T, M>(g);
+    const Stencil<T> stn = stencil<T, M>(C, B.f, g);
+    const double *sv = fstate + fid * kFT;
+    const FluxState s = flux_state(sv);
+    const d2 n = mk2(sv[29], sv[30]);
+    AS1 V2<T> *fout = (AS1 V2<T> *)(R.face == SOUTH ? B.fluxS : B.fluxW) + g.own * (size_t)C.NV;
+    double mf[4] = {0.0, 0.0, 0.0, 0.0};
+    if (C.nut > 0 && (n.x == 0.0 || n.y == 0.0)) {
+        const bool wtype = n.y == 0.0;
+        const int na = wtype ? C.nut : C.nvt, nb = wtype ? C.nvt : C.nut;
+        const double *qa = wtype ? C.qu : C.qv, *qb = wtype ? C.qv : C.qu;
+        const double ka = wtype ? n.x : n.y, kb = wtype ? n.x : -n.y;
+        const d2 unit = mk2(slope_unit<T, M>(C, g, 0), slope_unit<T, M>(C, g, 1));
+        AS3 char *tabN = tab, *tabT = tab + kTabN * na;
+        if (na <= 32 && nb <= 32) {
+            // both axes at once: lanes 0-31 take the normal one, 32-63 the tangential one
+            const int k = lane & 31;
+            const bool first = lane < 32;
+            if (k < (first ? na : nb)) {
+                const double q = first ? ka * qa[k] : kb * qb[k], c = q - (first ? s.U : s.V), E = exp(-s.lam * (c * c));
+                if (first) put_normal<T>(tabN + k * kTabN, s, unit, q, c, E);
+                else put_tangential<T>(tabT + k * kTabT, s, q, c, E);
+            }
+        } else {
+            if (lane < na) {
+                const double q = ka * qa[lane], c = q - s.U;
+                put_normal<T>(tabN + lane * kTabN, s, unit, q, c, exp(-s.lam * (c * c)));
+            }
+            if (lane < nb) {
+                const double q = kb * qb[lane], c = q - s.V;
+                put_tangential<T>(tabT + lane * kTabT, s, q, c, exp(-s.lam * (c * c)));
+            }
+        }
+        // the tables are private to this wavefront: order its LDS writes before its reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (wtype) flux_loop_tables<T, M, true>(C, stn, g, s, lane, sb, tabN, tabT, fout, mf);
+        else flux_loop_tables<T, M, false>(C, stn, g, s, lane, sb, tabN, tabT, fout, mf);
+    } else {
+        flux_loop_general<T, M>(C, stn, g, s, n, lane, sb, (AS3 double *)tab, nmax, fout, mf);
+    }
     wave_sum4(mf);
     if (lane == 0) {
-        d4 o = mk4(mf[0], mf[1], mf[2], mf[3]) + Lf * mk4(sv[24], sv[25], sv[26], sv[27]);
+        d4 o = mk4(mf[0], mf[1], mf[2], mf[3]) + sv[28] * mk4(sv[24], sv[25], sv[26], sv[27]);
         const d2 gl = to_global(mk2(o.s1, o.s2), n);
         o.s1 = gl.x; o.s2 = gl.y;
-        (L.face == SOUTH ? B.fmS : B.fmW)[g.own] = o;
+        (R.face == SOUTH ? B.fmS : B.fmW)[g.own] = o;
     }
 }
 
@@ -855,13 +1088,8 @@ __global__ void __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWallWa
     const FaceGeo g = face_geo(B, gi, gj, fid);
     const d2 n = B.normal[g.own * 2 + fid];
     const double L = B.side_length[g.own * 2 + fid];
-    const int mi = gi - C.G, mj = gj - C.G;
-    const bool wantQ = (fid == SOUTH) && (mj < C.nj);
-    const d4 cm = wantQ ? B.macro[(size_t)mi * C.nj + mj] : mk4(0, 0, 0, 1);
-
-    // reconstruction at the wall face (iFace) and the owner heat flux
+    // reconstruction at the wall face (iFace)
     P2<T> ff[NPT];
-    double acc[2] = {0.0, 0.0};
     const Stencil<T> stn = stencil<T>(C, B.f, g);
 #pragma unroll
     for (int k = 0; k < NPT; k++) {
@@ -870,20 +1098,7 @@ __global__ void __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWallWa
             d2 uv = face_velocity(C, v, n);
             P2<T> sgk;
             reconstruct<T>(C, stn, g, v, upwind(uv.x), ff[k], sgk);
-            if (wantQ) {
-                P2<T> fl, fr;
-                face_cells<T>(C, stn, v, fl, fr);
-                d2 e = C.quad[v];
-                double a = (double)fr.x, bq = (double)fr.y;
-                double cx = e.x - cm.s1, cy = e.y - cm.s2, t = (cx * cx + cy * cy) * a + bq / C.K;
-                acc[0] += 0.5 * (cx * t);
-                acc[1] += 0.5 * (cy * t);
-            }
         }
-    }
-    if (wantQ) {
-        block_sum<2>(acc, red);
-        if (threadIdx.x == 0) B.Q[(size_t)mi * C.nj + mj] = mk2(acc[0], acc[1]);
     }
     d4 wall = B.wall_prop[(size_t)ci * 4 + face];
     {
@@ -1105,6 +1320,24 @@ __device__ __forceinline__ void add_moments(const Consts &C, int v, T gx, T hx, 
     add_moments<T>(quad_at(C, v), gx, hx, m);
 }
 
+// Heat flux terms of one velocity about a cell's mean velocity (calcQ,
+// clKernel.c:480-543): c the peculiar velocity, c2 its square, rK = 1 / K.
+// The same rule on rounding as above.
+__device__ __forceinline__ double peculiar2(double cx, double cy) { return fma(cy, cy, cx * cx); }
+template <typename T>
+__device__ __forceinline__ void add_heat(double cx, double cy, double c2, double rK, T gx, T hx, double (&q)[2]) {
+#pragma clang fp contract(off)
+    const double t = fma(rK, (double)hx, c2 * (double)gx);
+    q[0] = fma(0.5, cx * t, q[0]);
+    q[1] = fma(0.5, cy * t, q[1]);
+}
+// the heat flux summed over the wavefront and stored: components 0 and 1 end in rows 0 and 1
+__device__ __forceinline__ void store_heat(d2 *dst, const double (&q)[2], int lane) {
+    const double a[4] = {q[0], q[1], 0.0, 0.0};
+    const double r = wave_sum4_rows(a);
+    if ((lane & 15) == 0 && lane < 32) ((double *)dst)[lane >> 4] = r;
+}
+
 // A cell's four moments summed over the wavefront (all 64 lanes active) and
 // stored: the first lane of row r writes component r.  The update, the ghost
 // fills and the per-call refresh all store through here, so a cell's
@@ -1125,12 +1358,20 @@ __global__ void __launch_bounds__(kT) k_cellmom(const FBlock *__restrict__ block
     const Consts &C = B.c;
     const long long cell = item - off[b];
     const P2<T> *F = (const P2<T> *)B.f + cell * C.NV;
-    double m[4] = {0.0, 0.0, 0.0, 0.0};
+    const int mi = (int)(cell / C.NJ) - C.G, mj = (int)(cell % C.NJ) - C.G;
+    const bool inner = mi >= 0 && mi < C.ni && mj >= 0 && mj < C.nj;      // ghost cells have no heat flux
+    const d4 p = inner ? B.macro[(size_t)mi * C.nj + mj] : mk4(0, 0, 0, 1);
+    const double rK = 1.0 / C.K;
+    double m[4] = {0.0, 0.0, 0.0, 0.0}, q[2] = {0.0, 0.0};
     for (int v = lane; v < C.NV; v += 64) {
         const P2<T> x = F[v];
-        add_moments<T>(C, v, x.x, x.y, m);
+        const d2 e = quad_at(C, v);
+        add_moments<T>(e, x.x, x.y, m);
+        const double cx = e.x - p.s1, cy = e.y - p.s2;
+        add_heat<T>(cx, cy, peculiar2(cx, cy), rK, x.x, x.y, q);
     }
     store_moments(B.cmom + cell, m, lane);
+    if (inner) store_heat(B.qnext + (size_t)mi * C.nj + mj, q, lane);
 }
 
 // ============================================================ k_update ====
@@ -1161,13 +1402,14 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const double A = B.area[c0];
     const d4 dW = ((B.fmS[c0] - B.fmS[c0 + 1]) + B.fmW[c0]) - B.fmW[c0 + C.NJ];
     const d4 p = to_primary(C, to_conserved(C, pold) + dW / A);
+    const d2 Q = B.qnext[cell];
     if (lane == 0) {
         B.macro_new[cell] = p;
         B.residual[cell] = pold;
+        B.Q[cell] = Q;
     }
     // UGKS_update (clUGKS.c:1189-1257)
     const double tau_old = relax_time(C, pold), tau = relax_time(C, p);
-    const d2 Q = B.Q[cell];
     const bool sep = C.nut > 0;
     double (*tab)[64] = tabs[wv];
     if (sep) {
@@ -1195,7 +1437,7 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const double Qx = uniform_d(Q.x), Qy = uniform_d(Q.y);
     const double urlo = uniform_d(rlo), urln = uniform_d(rln), uso = uniform_d(so), usn = uniform_d(sn);
     const double uhfo = uniform_d(hfo), uhfn = uniform_d(hfn), urA = uniform_d(rA), urden = uniform_d(rden);
-    const double uhtn = uniform_d(htn), uhto = uniform_d(hto);
+    const double uhtn = uniform_d(htn), uhto = uniform_d(hto), urK = uniform_d(1.0 / C.K);
     // this cell's velocities in f and in the four face fluxes: uniform bases, 32-bit lane offsets
     const long long NV = C.NV;
     AS1 V2<T> *fc = (AS1 V2<T> *)B.f + c0 * NV;
@@ -1209,7 +1451,7 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const int nvt = __builtin_amdgcn_readfirstlane(C.nvt);
     if (sep) { iu = lane / nvt; jv = lane - iu * nvt; diu = 64 / nvt; djv = 64 - diu * nvt; }
     bool nan_seen = false;
-    double mom[4] = {0.0, 0.0, 0.0, 0.0};
+    double mom[4] = {0.0, 0.0, 0.0, 0.0}, heat[2] = {0.0, 0.0};
     // the velocity and weight of the next iteration are loaded one iteration
     // ahead, and this velocity's f and face fluxes before its Maxwellians, so
     // the loads of an iteration overlap its arithmetic instead of stalling it
@@ -1225,7 +1467,7 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
             wnext = weight_at(C, vn);
         }
         const double ox = e.x - po1, oy = e.y - po2, nx = e.x - pn1, ny = e.y - pn2;
-        const double co = ox * ox + oy * oy, cn = nx * nx + ny * ny;
+        const double co = ox * ox + oy * oy, cn = peculiar2(nx, ny);
         double Eo, En;
         if (sep) {
             Eo = tab[0][iu] * tab[1][jv];
@@ -1250,11 +1492,13 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
         const T tg = (T)ng, th = (T)nh;
         if (isnan(tg) || isnan(th)) nan_seen = true;
         stream_store<T>(fc + v, V2<T>{tg, th});
-        // the new cell moments (the getAL / getAR inputs of the next step)
+        // the new cell's moments and heat flux (the next step's getAL / getAR and update inputs)
         add_moments<T>(e, tg, th, mom);
+        add_heat<T>(nx, ny, cn, urK, tg, th, heat);
     }
     if (nan_seen) B.flag[0] = ERR_NAN;
     store_moments(B.cmom + c0, mom, lane);
+    store_heat(B.qnext + cell, heat, lane);
 }
 
 // ============================================================ k_dt =========
@@ -1570,8 +1814,10 @@ struct ugks_step_plan {
     long long *d_face_off, *d_cell_off, *d_all_off;   // prefix offsets: interior faces, cells, all cells
     long long *d_tile_off;                              // prefix offsets of the update's 2 x 2 cell tiles
     long long nall, ntiles;
+    int nmax;                             // velocities on the longest axis of any block's tensor grid (at most 64)
     int fa_waves, fc_waves;               // workgroup size of the face passes, in wavefronts (1, 2 or 4)
     int method;                           // the blocks' common reconstruction method, -1 if they differ
+    d2 *d_qnext;                                        // heat flux of every block's cells, back to back
     d4 *d_cmom;                                         // cell moments of every block, back to back
     WallItem *d_walls;
     GhostItem *d_ghosts;
@@ -1599,8 +1845,9 @@ template <typename T, int FW, int M> void launch_faceA(ugks_step_plan *p, hipStr
                        p->d_blocks, (const FaceRec *)p->d_frec, (const int *)p->d_tmap, p->nfaces, p->d_fsum);
 }
 template <typename T, int FW, int M> void launch_faceC(ugks_step_plan *p, hipStream_t s) {
-    hipLaunchKernelGGL((k_faceC<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW), 0, s,
-                       p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces, (const double *)p->d_fstate);
+    hipLaunchKernelGGL((k_faceC<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
+                       FW * (kStenLds<T> + kTabBytes * p->nmax), s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
+                       (const double *)p->d_fstate, p->nmax);
 }
 // the face passes specialised for the plan's one reconstruction method (or generic)
 template <typename T, int FW> void faceA_m(ugks_step_plan *p, hipStream_t s) {
@@ -1638,7 +1885,7 @@ template <typename T, int NPT> int launch_step(ugks_step_plan *p, hipStream_t s,
         faceA<T>(p, s, p->fa_waves);
     if (ev) (void)hipEventRecord(ev[1], s);
     if (p->nfaces > 0)
-        hipLaunchKernelGGL(k_faceS, dim3(gt), dim3(kT), 0, s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
+        hipLaunchKernelGGL((k_faceS<T>), dim3(gt), dim3(kT), 0, s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
                            (const double *)p->d_fsum, p->d_fstate, (const DtState *)p->d_state);
     if (ev) (void)hipEventRecord(ev[2], s);
     if (p->nfaces > 0)
@@ -1725,7 +1972,7 @@ template <typename T> int autotune(ugks_step_plan *p, hipStream_t s, int reps, i
             const int fw = cand[c];
             // kC reads kA's results through kS: run the chain once, then time the kernel alone
             faceA<T>(p, s, which == 0 ? fw : p->fa_waves);
-            hipLaunchKernelGGL(k_faceS, dim3((unsigned)((p->nfaces + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks,
+            hipLaunchKernelGGL((k_faceS<T>), dim3((unsigned)((p->nfaces + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks,
                                (const FaceRec *)p->d_frec, p->nfaces, (const double *)p->d_fsum, p->d_fstate,
                                (const DtState *)p->d_state);
             (void)hipEventRecord(e0, s);
@@ -1886,7 +2133,7 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     for (int b = 0; b < nblocks; b++)
         if (p->host_blocks[b].c.nut > 64 || p->host_blocks[b].c.nvt > 64) {
             delete p; return ugks_rt::fail(-2, "step plan: more than 64 velocities per axis");
-        }
+        } else p->nmax = std::max(p->nmax, std::max(p->host_blocks[b].c.nut, p->host_blocks[b].c.nvt));
     p->nfaces = face_off[nblocks];
     if (p->nfaces >= (1LL << 31)) { delete p; return ugks_rt::fail(-2, "step plan: 2^31 or more interior faces"); }
     p->ncells = cell_off[nblocks];
@@ -1905,13 +2152,14 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     (void)alloc((void **)&p->d_all_off, sizeof(long long) * (nblocks + 1));
     (void)alloc((void **)&p->d_tile_off, sizeof(long long) * (nblocks + 1));
     (void)alloc((void **)&p->d_cmom, sizeof(d4) * (size_t)p->nall);
+    (void)alloc((void **)&p->d_qnext, sizeof(d2) * (size_t)p->ncells);
     (void)alloc((void **)&p->d_walls, sizeof(WallItem) * (walls.size() ? walls.size() : 1));
     (void)alloc((void **)&p->d_ghosts, sizeof(GhostItem) * ghosts.size());
     (void)alloc((void **)&p->d_state, sizeof(DtState) * ncases);
     (void)alloc((void **)&p->d_case_first, sizeof(int) * (ncases + 1));
     (void)alloc((void **)&p->d_maxbits, sizeof(unsigned long long) * nblocks);
     (void)alloc((void **)&p->d_max_dt, sizeof(double) * nblocks);
-    (void)alloc((void **)&p->d_fsum, sizeof(double) * kFS * (size_t)p->nfaces);
+    (void)alloc((void **)&p->d_fsum, sizeof(double) * kFSof(precision) * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_fstate, sizeof(double) * kFT * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_frec, sizeof(FaceRec) * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_tmap, sizeof(int) * (size_t)p->nfaces);
@@ -1928,7 +2176,10 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     }
     std::vector<unsigned long long> zeros(nblocks, 0ull);
     if (e == hipSuccess)
-        for (int b = 0; b < nblocks; b++) p->host_blocks[b].cmom = p->d_cmom + all_off[b];
+        for (int b = 0; b < nblocks; b++) {
+            p->host_blocks[b].cmom = p->d_cmom + all_off[b];
+            p->host_blocks[b].qnext = p->d_qnext + cell_off[b];
+        }
     if (e == hipSuccess) e = hipMemcpy(p->d_blocks, p->host_blocks.data(), bytes_blocks, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_face_off, face_off.data(), sizeof(long long) * (nblocks + 1), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_cell_off, cell_off.data(), sizeof(long long) * (nblocks + 1), hipMemcpyHostToDevice);
@@ -1965,7 +2216,7 @@ int ugks_step_plan_destroy(ugks_step_plan *p) {
     if (p->graph_exec) (void)hipGraphExecDestroy(p->graph_exec);
     if (p->graph) (void)hipGraphDestroy(p->graph);
     if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
-    void *ptrs[] = {p->d_blocks, p->d_face_off, p->d_cell_off, p->d_all_off, p->d_tile_off, p->d_cmom, p->d_walls, p->d_ghosts,
+    void *ptrs[] = {p->d_blocks, p->d_face_off, p->d_cell_off, p->d_all_off, p->d_tile_off, p->d_cmom, p->d_qnext, p->d_walls, p->d_ghosts,
                     p->d_state, p->d_case_first, p->d_maxbits, p->d_max_dt, p->d_fsum, p->d_fstate, p->d_frec,
                     p->d_tmap, p->d_udf_blocks};
     for (void *q : ptrs)
@@ -2291,6 +2542,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     for (int b = 0; b < nblocks; b++)
         if (host[b].c.nut > 64 || host[b].c.nvt > 64)
             return ugks_rt::fail(-2, "step noalloc: more than 64 velocities per axis");
+        else P.nmax = std::max(P.nmax, std::max(host[b].c.nut, host[b].c.nvt));
     if (T.off[0][nblocks] >= (1LL << 31)) return ugks_rt::fail(-2, "step noalloc: 2^31 or more interior faces");
     P.npt = npt;
     P.nfaces = T.off[0][nblocks];
@@ -2303,26 +2555,31 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     P.nghost_items = T.nghost;
     P.nudf = T.nudf;
     P.udf_wl = udf_wl;
-    // carve the working memory: 256-byte aligned regions, refused if they do not fit
-    size_t at = 0;
-    bool fits = true;
-    auto carve = [&](size_t bytes) {
+    // carve the working memory: 256-byte aligned regions, refused if they do not fit.
+    // A case's size is accounted with 128 bytes of face sums per face and no
+    // heat fluxes, so the same cases are taken as ever; the layout (96 or 104
+    // bytes per face and 16 per cell) is never larger where the limit is near.
+    size_t at = 0, counted = 0;
+    auto carve = [&](size_t bytes, size_t as) {
         const size_t here = at;
         at = (at + bytes + 255) & ~(size_t)255;
-        if (at > kNoAllocBytes) fits = false;
+        counted = (counted + as + 255) & ~(size_t)255;
         return here;
     };
-    const size_t o_blocks = carve(sizeof(FBlock) * nblocks), o_off = carve(sizeof(long long) * 4 * (nblocks + 1)),
-                 o_walls = carve(sizeof(WallItem) * 4 * nblocks), o_ghosts = carve(sizeof(GhostItem) * 4 * nblocks),
-                 o_udf = carve(sizeof(int) * nblocks), o_case = carve(sizeof(int) * 2), o_state = carve(sizeof(DtState)),
-                 o_maxbits = carve(sizeof(unsigned long long) * nblocks), o_maxdt = carve(sizeof(double) * nblocks),
-                 o_cmom = carve(sizeof(d4) * (size_t)P.nall), o_fsum = carve(sizeof(double) * kFS * (size_t)P.nfaces),
-                 o_fstate = carve(sizeof(double) * kFT * (size_t)P.nfaces),
-                 o_frec = carve(sizeof(FaceRec) * (size_t)P.nfaces), o_tmap = carve(sizeof(int) * (size_t)P.nfaces);
-    if (!fits) {
+    auto region = [&](size_t bytes) { return carve(bytes, bytes); };
+    const size_t o_blocks = region(sizeof(FBlock) * nblocks), o_off = region(sizeof(long long) * 4 * (nblocks + 1)),
+                 o_walls = region(sizeof(WallItem) * 4 * nblocks), o_ghosts = region(sizeof(GhostItem) * 4 * nblocks),
+                 o_udf = region(sizeof(int) * nblocks), o_case = region(sizeof(int) * 2), o_state = region(sizeof(DtState)),
+                 o_maxbits = region(sizeof(unsigned long long) * nblocks), o_maxdt = region(sizeof(double) * nblocks),
+                 o_cmom = region(sizeof(d4) * (size_t)P.nall),
+                 o_fsum = carve(sizeof(double) * kFSof(precision) * (size_t)P.nfaces, sizeof(double) * 16 * (size_t)P.nfaces),
+                 o_qnext = carve(sizeof(d2) * (size_t)P.ncells, 0),
+                 o_fstate = region(sizeof(double) * kFT * (size_t)P.nfaces),
+                 o_frec = region(sizeof(FaceRec) * (size_t)P.nfaces), o_tmap = region(sizeof(int) * (size_t)P.nfaces);
+    if (std::max(at, counted) > kNoAllocBytes) {
         char msg[200];
         snprintf(msg, sizeof msg, "step noalloc: the case needs %zu bytes of working memory; the allocation-free "
-                                  "step has %zu per GPU", at, kNoAllocBytes);
+                                  "step has %zu per GPU", std::max(at, counted), kNoAllocBytes);
         return ugks_rt::fail(-2, msg);
     }
     unsigned char *base = nullptr;
@@ -2347,6 +2604,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     P.d_tmap = (int *)(base + o_tmap);
     for (int b = 0; b < nblocks; b++) {
         host[b].cmom = P.d_cmom + T.off[2][b];
+        host[b].qnext = (d2 *)(base + o_qnext) + T.off[1][b];
         hipLaunchKernelGGL(k_put_block, dim3(1), dim3(64), 0, s, host[b], P.d_blocks + b);
     }
     hipLaunchKernelGGL(k_put_tables, dim3(1), dim3(kT), 0, s, T, off, P.d_walls, P.d_ghosts, P.d_udf_blocks,

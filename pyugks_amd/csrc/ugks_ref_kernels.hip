@@ -237,7 +237,7 @@ __device__ __forceinline__ void iface_face(const Consts &C, const d2 *__restrict
         const d2 cm = centre[cidx(C, gi + di * (o0 + MID * os), gj + dj * (o0 + MID * os))];
         dist[delta] = length(mside - cm);
         dlen[delta] = length(c1 - c0);
-        rdist[delta] = 1.0 / dist[delta];
+        rdist[delta] = (1.0 / 6.0) / dist[delta];
     }
     const d2 *fc = F + fidx(C, gi, gj, 0);
     const size_t out0 = fidx(C, gi, gj, 0);
@@ -259,8 +259,9 @@ __device__ __forceinline__ void iface_face(const Consts &C, const d2 *__restrict
         } else if constexpr (METHOD == 1) {
             // the reference's WENO5 (clFunctions.c:268-312) rearranged to one
             // quotient per component; it agrees with the literal form to rounding
-            weno5_slope_pair(fs[0].x, fs[1].x, fs[2].x, fs[3].x, fs[4].x, fs[0].y, fs[1].y, fs[2].y, fs[3].y, fs[4].y,
-                             delta ? rdist[1] : rdist[0], sig.x, sig.y);
+            weno5_q_pair(fs[0].x, fs[1].x, fs[2].x, fs[3].x, fs[4].x, fs[0].y, fs[1].y, fs[2].y, fs[3].y, fs[4].y,
+                         sig.x, sig.y);
+            sig = (delta ? rdist[1] : rdist[0]) * sig;
         } else {
             sig.x = nnd(fs[0].x, fs[1].x, fs[2].x, dst);
             sig.y = nnd(fs[0].y, fs[1].y, fs[2].y, dst);
