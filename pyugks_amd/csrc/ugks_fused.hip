@@ -380,120 +380,75 @@ __device__ __forceinline__ void reconstruct(const Consts &C, const Stencil<T> &s
 }
 
 #define AS3 __attribute__((address_space(3)))
-// LDS bytes of one wavefront's stencil staging: all 2R stencil cells (both
-// upwind choices) of 64 velocities.  FP64 only: a lane's (g, h) pair of floats
-// is 8 bytes, a size the LDS loads lack.  The flux pass stages its stencils
-// this way; the moment pass, which has no store in its loop and runs at a
-// higher occupancy, measured faster with plain loads.
-template <typename T> constexpr int kStenRow = 64 * (int)sizeof(P2<T>);
-template <typename T> constexpr bool kStenViaLds = sizeof(T) == 8;
-template <typename T> constexpr int kStenLds = kStenViaLds<T> ? 6 * kStenRow<T> : 16;
-
-// Loads of the 2R stencil cells of the velocities at byte offset vb, issued
-// straight into the wavefront's LDS buffer lb (no registers held while they
-// are in flight): cell r of lane l lands at lb + r * kStenRow + l * sizeof(P2).
-template <typename T, int M>
-__device__ __forceinline__ void stencil_dma(const Consts &C, const Stencil<T> &st, unsigned vb, AS3 char *lb) {
-    constexpr int sz = 16;   // one (g, h) pair of doubles per lane
-    const int ncell = method_of<M>(C) == 1 ? 6 : 4;
-    // The row addresses are formed again at every call, by scalar adds.
-    // Hoisted out of the velocity loop, the six 64-bit global and six LDS
-    // row addresses took 18 scalar registers the flux pass does not have:
-    // they were spilled to vector lanes and read back with v_readlane
-    // (vector instructions, each followed by wait states) in every iteration.
-    unsigned sb = st.sb, lds = (unsigned)(size_t)lb;
-    __asm__ volatile("" : "+s"(sb), "+s"(lds));
-#pragma unroll
-    for (int r = 0; r < 6; r++) {
-        if (r < ncell) {
-            const AS1 char *src = st.base + r * sb;
-            __builtin_amdgcn_global_load_lds((const AS1 void *)(src + vb), (AS3 void *)(size_t)(lds + r * kStenRow<T>), sz,
-                                             0, 0);
-        }
-    }
-}
-template <typename T> __device__ __forceinline__ P2<T> lld(const AS3 char *p) {
-    const V2<T> x = *(const AS3 V2<T> *)p;
-    return P2<T>{x.x, x.y};
-}
-// the stencil of this lane's velocity from the staging buffer, in stencil
-// index order for upwind choice delta (cells 0..4 for delta = 1, 5..1 for 0)
-template <typename T, int M>
-__device__ __forceinline__ void stencil_read(const Consts &C, const AS3 char *lb, int lane, int delta, StenVals<T> &x) {
-    constexpr int row = kStenRow<T>;
-    const int last = method_of<M>(C) == 1 ? 5 : 3;
-    const AS3 char *p = lb + lane * (int)sizeof(P2<T>) + (delta ? 0 : last * row);
-    const int s = delta ? row : -row;
-    x.s0 = lld<T>(p);
-    x.s1 = lld<T>(p + s);
-    x.s2 = lld<T>(p + 2 * s);
-    if (method_of<M>(C) == 1) {
-        x.s3 = lld<T>(p + 3 * s);
-        x.s4 = lld<T>(p + 4 * s);
-    } else {
-        x.s3 = x.s4 = x.s2;
-    }
-}
-
 // to_local with its fused operations written out (the mixed plan keeps one order of operations)
 __device__ __forceinline__ d2 to_face(d2 m, d2 n) { return d2{fma(m.y, n.y, m.x * n.x), fma(m.y, n.x, -(m.x * n.y))}; }
 
-// Waits around the staging buffer, written out: the compiler's own tracking of
-// loads into LDS loses them where a loop it has peeled joins its header (the
-// buffer was then read before the loads had landed).  The memory clobbers
-// keep its LDS reads between the two.
-__device__ __forceinline__ void stencil_landed() { __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-__device__ __forceinline__ void stencil_consumed() { __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+// Where a face pass takes its velocities from: the velocity table (one entry
+// loaded an iteration ahead), or on a tensor grid the two axes in LDS.  The
+// vector L1 spends 16 cycles on a wavefront's 16-byte loads and as much on its
+// 8-byte ones, and the moment pass kept it busy nearly all the time: without
+// the table's load it went 0.75 -> 0.68 ms FP64 and 0.56 -> 0.51 ms mixed (2 x 2
+// blocks of 128^2 cells, 33^2 velocities, WENO5).
+template <bool WEIGHT> struct TableVelocities {
+    const Consts &C;
+    d2 e;
+    double w = 0.0, wc = 0.0;       // the next velocity's weight, this one's
+    __device__ __forceinline__ TableVelocities(const Consts &c, int lane) : C(c) { load(lane < c.NV ? lane : 0); }
+    __device__ __forceinline__ void load(int v) {
+        e = quad_at(C, v);
+        if constexpr (WEIGHT) w = weight_at(C, v);
+    }
+    __device__ __forceinline__ d2 next() { wc = w; return e; }
+    // velocity v + 64, or v again on the last round: no branch
+    __device__ __forceinline__ void prefetch(int v) { load(v + 64 < C.NV ? v + 64 : v); }
+};
+struct AxisVelocities {
+    const AS3 double *qu, *qv;      // this lane's entries
+    const AS3 double *end;
+    int nvt, du, dv;
+    // tab: LDS for nut + nvt values of this wavefront
+    __device__ __forceinline__ AxisVelocities(const Consts &C, AS3 double *tab, int lane) {
+        const int nut = C.nut;
+        nvt = __builtin_amdgcn_readfirstlane(C.nvt);
+        if (lane < nut) tab[lane] = C.qu[lane];
+        if (lane < nvt) tab[nut + lane] = C.qv[lane];
+        // private to this wavefront: order its LDS writes before its reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int iu = lane / nvt;
+        qu = tab + iu;
+        qv = tab + nut + (lane - iu * nvt);
+        end = tab + nut + nvt;
+        du = 64 / nvt;
+        dv = 64 - du * nvt;
+    }
+    __device__ __forceinline__ d2 next() {
+        const d2 x = d2{*qu, *qv};
+        qu += du; qv += dv;
+        if (qv >= end) { qv -= nvt; qu++; }
+        return x;
+    }
+    __device__ __forceinline__ void prefetch(int) {}
+};
 
 // Velocity loop of a wavefront-per-face pass, v = lane, lane + 64, ...: the
-// body gets the global velocity e, its weight w, the face-frame velocity uv,
-// the upwind choice and the stencil.  The stencil of the next velocity is
-// loaded into the wavefront's LDS buffer lb while the body of this one runs
-// (both upwind choices, so the loads need not wait for the next velocity);
-// the velocity and weight are loaded one iteration ahead into registers.
-template <typename T, int M, bool LDS, typename Body>
-__device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stencil<T> &st, d2 n, int lane, AS3 char *lb,
-                                                   Body body) {
-    static_assert(!LDS || kStenViaLds<T>, "LDS stencil staging needs FP64 pairs");
-    if (lane >= C.NV) return;
-    d2 e = quad_at(C, lane);
-    double w = weight_at(C, lane);
-    unsigned vb = (unsigned)lane * (unsigned)sizeof(P2<T>);
-    if constexpr (LDS) stencil_dma<T, M>(C, st, vb, lb);
+// body gets the global velocity e, the face-frame velocity uv, the upwind
+// choice and the stencil.
+template <typename T, int M, typename Vel, typename Body>
+__device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stencil<T> &st, d2 n, int lane, Vel &vel, Body body) {
     for (int v = lane; v < C.NV; v += 64) {
-        const d2 ec = e;
-        const double wc = w;
-        const d2 uv = to_face(ec, n);
-
+        const d2 e = vel.next();
+        const d2 uv = to_face(e, n);
         const int delta = upwind(uv.x);
+        vel.prefetch(v);
         StenVals<T> cur;
-        // the next velocity's table entries, or this one's again on the last
-        // round: the loads then need no branch (and no register copies around
-        // one).  The stencil loads into LDS stay conditional, so none is still
-        // in flight when the wavefront leaves the loop.
-        const int vn = v + 64 < C.NV ? v + 64 : v;
-        if constexpr (LDS) {
-            stencil_landed();
-            stencil_read<T, M>(C, lb, lane, delta, cur);
-            stencil_consumed();   // the reads have returned before the next loads overwrite the buffer
-            e = quad_at(C, vn);
-            w = weight_at(C, vn);
-            if (v + 64 < C.NV) {
-                vb += 64u * (unsigned)sizeof(P2<T>);
-                stencil_dma<T, M>(C, st, vb, lb);
-            }
-        } else {
-            e = quad_at(C, vn);
-            w = weight_at(C, vn);
-            stencil_load<T, M>(C, st, v, delta, cur);
-        }
-        body(v, ec, wc, uv, delta, cur);
+        stencil_load<T, M>(C, st, v, delta, cur);
+        body(v, e, uv, delta, cur);
     }
 }
 
 // ============================================================ face passes ==
-// Faces are numbered so that neighbouring ids share stencil cells: S faces
-// column by column (j fastest), W faces row by row (i fastest).
 // Per interior face: (A) one wavefront reconstructs f at the face for every
 // velocity and sums the raw face moments (the conserved moments of
 // getFaceCons and the third-order ones the face heat flux of calcFaceQ needs,
@@ -501,14 +456,12 @@ __device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stenci
 // cell moments (getAL/getAR) and the geometry into the face state (getPLR,
 // initMacroFlux, calcFaceQ); (C) one wavefront rebuilds the face values and
 // forms the per-velocity flux (distFlux) and the macro flux (macroFlux).
-// Face ids: per block, S faces then W faces (walls excluded).
+// Face ids: per block, in tiles (face_loc_tiled; walls excluded).
 //
 // The FP64 plan's face sums, with e the velocity and E = |e|^2: 0 g, 1-2 e g,
 // 3 ex^2 g, 4 ey^2 g, 5 ex ey g, 6-7 E e g, 8 h, 9-10 e h.  The heat flux only
 // needs the contracted third moment, which rotates as a vector, so no velocity
-// is rotated in the loop and 11 sums do.  (With the shorter WENO5 and the cell's
-// heat flux left to the update the pass went 0.85 -> 0.75 ms on 2 x 2 blocks of
-// 128^2 cells with 33^2 velocities.)  The mixed plan's sums are the face
+// is rotated in the loop and 11 sums do.  The mixed plan's sums are the face
 // frame's, 0 g, 1 u g, 2 w g, 3 u^2 g, 4 w^2 g, 5 u w g, 6 u^3 g, 7 w^3 g,
 // 8 u w^2 g, 9 u^2 w g, 10 h, 11 u h, 12 w h: its f is rounded to FP32 every
 // step, where a last-bit difference in these sums would now and then turn a
@@ -518,30 +471,18 @@ inline int kFSof(int precision) { return precision == UGKS_FP64 ? kFS<double> : 
 constexpr int kFT = 32;                                               // face state per face
 
 struct FaceLoc { int face, mi, mj, gi, gj; };
-__device__ __forceinline__ FaceLoc face_loc(const FBlock &B, long long loc) {
-    const Consts &C = B.c;
-    FaceLoc f;
-    if (loc < B.nS) { f.face = SOUTH; f.mi = (int)(loc / B.nSj); f.mj = (int)(loc % B.nSj) + B.ob_S; }
-    else { long long r = loc - B.nS; f.face = WEST; f.mj = (int)(r / B.nWi); f.mi = (int)(r % B.nWi) + B.ob_W; }
-    f.gi = f.mi + C.G;
-    f.gj = f.mj + C.G;
-    return f;
-}
-// the face_loc index of a face
-__device__ __forceinline__ long long face_index(const FBlock &B, const FaceLoc &f) {
-    return f.face == SOUTH ? (long long)f.mi * B.nSj + (f.mj - B.ob_S)
-                           : B.nS + (long long)f.mj * B.nWi + (f.mi - B.ob_W);
-}
-
-// The moment pass walks a block's faces in tiles of kTileI x kTileJ cells
+// The face passes walk a block's faces in tiles of kTileI x kTileJ cells
 // (tiles j-fastest): each tile's S faces (j fastest), then its W faces (i
 // fastest).  The S faces form an ni x nSj rectangle (mi, mj - ob_S), the W faces
 // an nWi x nj one (mi - ob_W, mj); the same tile grid cuts both, so the two
 // kinds of face that read a cell's stencil data run at about the same time
-// and share it in the caches.  (The flux pass measured faster in the plain
-// order, and it and the state pass keep it; the moment pass writes each
-// face's sums at the face's plain index.)  loc < 2^31 (checked on the host).
-constexpr int kTileI = 4, kTileJ = 16;
+// and share it in the caches.  A tile's 128 faces are one run of workgroups on
+// one XCD (xcd_remap).  Against all S faces first and then all W faces the flux
+// pass takes 3.33 instead of 3.47 ms on an uneven batch of 16 cases and 7.9 instead
+// of 8.3 on the channel (FP64); rows of 32 or of a whole block, 4 x 16, 8 x 16
+// (also as one run), 16 x 16 and 2 x 8 tiles are level or slower.  loc < 2^31
+// (checked on the host).
+constexpr int kTileI = 8, kTileJ = 8;
 __device__ __forceinline__ FaceLoc face_loc_tiled(const FBlock &B, long long loc64) {
     const Consts &C = B.c;
     const int loc = (int)loc64;
@@ -597,35 +538,34 @@ __device__ __forceinline__ FaceGeo face_geo_of(const FaceRec &r, const Consts &C
     return g;
 }
 
-// rec[fid]: the face of plain index fid (per block, S faces then W faces);
-// tmap[fid]: the plain index of the moment pass's item fid (tiled order)
+// rec[fid]: face fid (per block, in tiled order)
 __global__ void __launch_bounds__(kT) k_facerec(const FBlock *__restrict__ blocks, const long long *__restrict__ off,
-                                                int nb, long long nfaces, FaceRec *__restrict__ rec,
-                                                int *__restrict__ tmap) {
+                                                int nb, long long nfaces, FaceRec *__restrict__ rec) {
     const long long fid = (long long)blockIdx.x * kT + threadIdx.x;
     if (fid >= nfaces) return;
     const int b = find_block(off, nb, fid);
     const FBlock &B = blocks[b];
     const long long loc = fid - off[b];
-    const FaceLoc L = face_loc(B, loc);
+    const FaceLoc L = face_loc_tiled(B, loc);
     const FaceGeo g = face_geo(B, L.gi, L.gj, L.face);
     FaceRec r;
     r.b = b; r.face = L.face; r.gi = L.gi; r.gj = L.gj;
 #pragma unroll
     for (int k = 0; k < 2; k++) { r.dist[k] = g.dist[k]; r.rdist[k] = g.rdist[k]; r.rd1[k] = g.rd1[k]; }
     rec[fid] = r;
-    tmap[fid] = (int)(off[b] + face_index(B, face_loc_tiled(B, loc)));
 }
 
+constexpr int kAxisBytes = 16;     // LDS bytes per wavefront and grid value of the longer axis (both axes)
 template <typename T, int FW, int M>
 __global__ void __launch_bounds__(64 * FW) k_faceA(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
-                                                   const int *__restrict__ tmap, long long nfaces,
-                                                   double *__restrict__ fsum) {
-    const long long fid = xcd_remap(blockIdx.x, gridDim.x) * FW + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+                                                   long long nfaces, double *__restrict__ fsum, int nmax) {
+    extern __shared__ __attribute__((aligned(16))) char fa_lds[];       // per wavefront: the velocity axes
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const long long fid = xcd_remap(blockIdx.x, gridDim.x) * FW + wv;
     if (fid >= nfaces) return;
+    AS3 char *axes = (AS3 char *)fa_lds + wv * (kAxisBytes * nmax);
     const int lane = threadIdx.x & 63;
-    const long long sid = tmap[fid];                          // where the state pass looks for this face
-    const FaceRec R = recs[sid];
+    const FaceRec R = recs[fid];
     const FBlock &B = blocks[R.b];
     const Consts &C = B.c;
     FaceGeo g = face_geo_of(R, C);
@@ -636,16 +576,7 @@ __global__ void __launch_bounds__(64 * FW) k_faceA(const FBlock *__restrict__ bl
     double a[4 * NR];
 #pragma unroll
     for (int q = 0; q < 4 * NR; q++) a[q] = 0.0;
-    if (lane < C.NV) {
-        d2 e = quad_at(C, lane);
-        for (int v = lane; v < C.NV; v += 64) {
-            const d2 ec = e;
-            const double un = fma(ec.y, n.y, ec.x * n.x);
-            const int delta = upwind(un);
-            // the next velocity, or this one again on the last round: no branch
-            e = quad_at(C, v + 64 < C.NV ? v + 64 : v);
-            StenVals<T> sv;
-            stencil_load<T, M>(C, stn, v, delta, sv);
+    auto add = [&](int, d2 ec, d2 uv, int delta, const StenVals<T> &sv) __attribute__((always_inline)) {
             P2<T> ff, sg;
             reconstruct_from<T, M>(C, g, delta, sv, ff, sg);
             const double gg = (double)ff.x, hh = (double)ff.y;
@@ -656,21 +587,27 @@ __global__ void __launch_bounds__(64 * FW) k_faceA(const FBlock *__restrict__ bl
                 a[6] = fma(x, Eg, a[6]); a[7] = fma(y, Eg, a[7]);
                 a[8] += hh; a[9] = fma(x, hh, a[9]); a[10] = fma(y, hh, a[10]);
             } else {
-                const double u = un, w = fma(ec.y, n.x, -(ec.x * n.y));
+                const double u = uv.x, w = uv.y;
                 const double ug = u * gg, wg = w * gg, uug = u * ug, wwg = w * wg;
                 a[0] += gg; a[1] += ug; a[2] += wg;
                 a[3] += uug; a[4] += wwg; a[5] += u * wg;
                 a[6] += u * uug; a[7] += w * wwg; a[8] += u * wwg; a[9] += w * uug;
                 a[10] += hh; a[11] += u * hh; a[12] += w * hh;
             }
-        }
+    };
+    if (C.nut > 0) {
+        AxisVelocities vel(C, (AS3 double *)axes, lane);
+        face_velocity_loop<T, M>(C, stn, n, lane, vel, add);
+    } else {
+        TableVelocities<false> vel(C, lane);
+        face_velocity_loop<T, M>(C, stn, n, lane, vel, add);
     }
     // row r of the wavefront gets the totals of sums NR r .. NR r + NR - 1; its first lane stores them
     double t[NR];
     wave_sum_rows<NR>(a, t);
     if ((lane & 15) == 0) {
         const int k = NR * (lane >> 4);
-        double *o = fsum + sid * kFS<T> + k;
+        double *o = fsum + fid * kFS<T> + k;
 #pragma unroll
         for (int q = 0; q < NR; q++)
             if (k + q < kFS<T>) o[q] = t[q];
@@ -828,16 +765,20 @@ __device__ __forceinline__ void put_tangential(AS3 char *p, const FluxState &s, 
 // fixed reconstruction run six (80 VGPRs; WENO5 spills 4 registers there and
 // is still faster than at five); the others are left to the compiler
 template <typename T, int M> constexpr int kFaceCWaves = (sizeof(T) == 4 && M >= 0) ? 6 : 1;
-// the FP64 flux stores one iteration late (the FP32 variant would spill more at six waves)
-template <typename T> constexpr bool kDeferStore = sizeof(T) == 8;
+// The FP64 flux is stored one iteration late, so the wait for an iteration's
+// loads does not also wait for the store before them (the FP32 variant would
+// spill more at six waves).  Plain stencil loads: staged through LDS by
+// 16-byte LDS loads an iteration ahead, as this pass once did, the buffer costs
+// the waves that hide as much (uneven batch of 16 cases 3.65 -> 3.47 ms without
+// it, 64^2 cells 34.5 -> 32.4 us, 2 x 2 blocks of 128^2 level).
+template <typename T> constexpr bool kDeferStore = sizeof(T) == 8 ;
 
 // Velocity loop of one face through the tables.  WT: the normal runs along u
 // (the slow velocity index), else along v (the fast one).  mf collects the
 // macro flux sums.
 template <typename T, int M, bool WT>
 __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, int lane,
-                                                 AS3 char *sb, AS3 char *tabN, AS3 char *tabT, AS1 V2<T> *fout, double (&mf)[4]) {
-    constexpr bool LDS = kStenViaLds<T>;
+                                                 AS3 char *tabN, AS3 char *tabT, AS1 V2<T> *fout, double (&mf)[4]) {
     const int NV = C.NV, nvt = __builtin_amdgcn_readfirstlane(C.nvt);
     if (lane >= NV) return;
     // LDS addresses of this lane's slow and fast table entries, advanced without division
@@ -846,8 +787,6 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
     AS3 char *ps = (WT ? tabN : tabT) + iu0 * ss, *pf = (WT ? tabT : tabN) + jv0 * sf;
     AS3 char *const pend_f = (WT ? tabT : tabN) + nvt * sf;
     double w = weight_at(C, lane);
-    unsigned vb = (unsigned)lane * (unsigned)sizeof(P2<T>);
-    if constexpr (LDS) stencil_dma<T, M>(C, stn, vb, sb);
     V2<T> pend = V2<T>{T(0), T(0)};
     int last = -1;
     for (int v = lane; v < NV; v += 64) {
@@ -857,20 +796,8 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
         const int delta = upwind(ux);
         const double wc = w;
         StenVals<T> cur;
-        const int vn = v + 64 < NV ? v + 64 : v;
-        if constexpr (LDS) {
-            stencil_landed();
-            stencil_read<T, M>(C, sb, lane, delta, cur);
-            stencil_consumed();   // the reads have returned before the next loads overwrite the buffer
-            w = weight_at(C, vn);
-            if (v + 64 < NV) {
-                vb += 64u * (unsigned)sizeof(P2<T>);
-                stencil_dma<T, M>(C, stn, vb, sb);
-            }
-        } else {
-            w = weight_at(C, vn);
-            stencil_load<T, M>(C, stn, v, delta, cur);
-        }
+        w = weight_at(C, v + 64 < NV ? v + 64 : v);
+        stencil_load<T, M>(C, stn, v, delta, cur);
         if constexpr (kDeferStore<T>) {
             if (v >= 64) stream_store<T>(vslot<T>(fout, v - 64), pend);
             last = v;
@@ -927,7 +854,7 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
 // not depend on the frame): Ei[v / nvt] * Ej[v % nvt].
 template <typename T, int M>
 __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, d2 n, int lane,
-                                                  AS3 char *sb, AS3 double *Ei, int nmax, AS1 V2<T> *fout, double (&mf)[4]) {
+                                                  AS3 double *Ei, int nmax, AS1 V2<T> *fout, double (&mf)[4]) {
     const bool tensor = sizeof(T) == 8 && C.nut > 0;
     AS3 double *Ej = Ei + nmax;
     if (tensor) {
@@ -950,7 +877,9 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
     // next, so the wait for the loads issued there does not also wait for it
     V2<T> pend = V2<T>{T(0), T(0)};
     int last = -1;
-    face_velocity_loop<T, M, kStenViaLds<T>>(C, stn, n, lane, sb, [&](int v, d2, double wv, d2 uv, int delta, const StenVals<T> &stv) __attribute__((always_inline)) {
+    TableVelocities<true> vel(C, lane);
+    face_velocity_loop<T, M>(C, stn, n, lane, vel, [&](int v, d2, d2 uv, int delta, const StenVals<T> &stv) __attribute__((always_inline)) {
+        const double wv = vel.wc;
         if constexpr (kDeferStore<T>) {
             if (v >= 64) stream_store<T>(fout + (v - 64), pend);
             last = v;
@@ -993,13 +922,12 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
 template <typename T, int FW, int M>
 __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kFaceCWaves<T, M>))) k_faceC(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
                                                    long long nfaces, const double *__restrict__ fstate, int nmax) {
-    // per wavefront: the stencil staging buffer, then the tables
-    extern __shared__ __attribute__((aligned(16))) char fc_lds[];
+    extern __shared__ __attribute__((aligned(16))) char fc_lds[];       // per wavefront: the tables
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const long long fid = xcd_remap(blockIdx.x, gridDim.x) * FW + wv;
     if (fid >= nfaces) return;
     const int lane = threadIdx.x & 63;
-    AS3 char *sb = (AS3 char *)fc_lds + wv * (kStenLds<T> + kTabBytes * nmax), *tab = sb + kStenLds<T>;
+    AS3 char *tab = (AS3 char *)fc_lds + wv * (kTabBytes * nmax);
     const FaceRec R = recs[fid];
     const FBlock &B = blocks[R.b];
     const Consts &C = B.c;
@@ -1041,10 +969,10 @@ __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kF
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (wtype) flux_loop_tables<T, M, true>(C, stn, g, s, lane, sb, tabN, tabT, fout, mf);
-        else flux_loop_tables<T, M, false>(C, stn, g, s, lane, sb, tabN, tabT, fout, mf);
+        if (wtype) flux_loop_tables<T, M, true>(C, stn, g, s, lane, tabN, tabT, fout, mf);
+        else flux_loop_tables<T, M, false>(C, stn, g, s, lane, tabN, tabT, fout, mf);
     } else {
-        flux_loop_general<T, M>(C, stn, g, s, n, lane, sb, (AS3 double *)tab, nmax, fout, mf);
+        flux_loop_general<T, M>(C, stn, g, s, n, lane, (AS3 double *)tab, nmax, fout, mf);
     }
     wave_sum4(mf);
     if (lane == 0) {
@@ -1827,10 +1755,9 @@ struct ugks_step_plan {
     DtState *d_state;                   // [ncases]
     int *d_case_first;                  // [ncases + 1] first block of each case
     double *d_fsum, *d_fstate;          // per interior face: raw sums, face state
-    FaceRec *d_frec;                    // per interior face: block, side, owner, distances (plain order)
+    FaceRec *d_frec;                    // per interior face: block, side, owner, distances
     int *d_udf_blocks;                  // blocks whose wall values are re-evaluated every step
     int nudf, udf_wl;                   // their count and largest wall length
-    int *d_tmap;                        // moment-pass item -> plain face index (tiled order)
     hipStream_t cap_stream;             // stream the step graph is captured on
     hipGraph_t graph;
     hipGraphExec_t graph_exec;
@@ -1841,12 +1768,13 @@ struct ugks_step_plan {
 
 namespace {
 template <typename T, int FW, int M> void launch_faceA(ugks_step_plan *p, hipStream_t s) {
-    hipLaunchKernelGGL((k_faceA<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW), 0, s,
-                       p->d_blocks, (const FaceRec *)p->d_frec, (const int *)p->d_tmap, p->nfaces, p->d_fsum);
+    hipLaunchKernelGGL((k_faceA<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
+                       FW * (kAxisBytes * p->nmax), s, p->d_blocks, (const FaceRec *)p->d_frec,
+                       p->nfaces, p->d_fsum, p->nmax);
 }
 template <typename T, int FW, int M> void launch_faceC(ugks_step_plan *p, hipStream_t s) {
     hipLaunchKernelGGL((k_faceC<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
-                       FW * (kStenLds<T> + kTabBytes * p->nmax), s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
+                       FW * kTabBytes * p->nmax, s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
                        (const double *)p->d_fstate, p->nmax);
 }
 // the face passes specialised for the plan's one reconstruction method (or generic)
@@ -1918,7 +1846,7 @@ template <typename T> int refresh_moments(ugks_step_plan *p, hipStream_t s) {
                        p->d_all_off, p->nb, p->nall);
     if (p->nfaces > 0)
         hipLaunchKernelGGL(k_facerec, dim3((unsigned)((p->nfaces + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks,
-                           p->d_face_off, p->nb, p->nfaces, p->d_frec, p->d_tmap);
+                           p->d_face_off, p->nb, p->nfaces, p->d_frec);
     hipLaunchKernelGGL(k_flipidx, dim3((unsigned)((4 * p->nb + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks, p->nb);
     return ugks_rt::check_launch("ugks_step: cell moments, face records and join corners");
 }
@@ -2162,7 +2090,6 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     (void)alloc((void **)&p->d_fsum, sizeof(double) * kFSof(precision) * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_fstate, sizeof(double) * kFT * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_frec, sizeof(FaceRec) * (size_t)p->nfaces);
-    (void)alloc((void **)&p->d_tmap, sizeof(int) * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_udf_blocks, sizeof(int) * (udf_blocks.size() ? udf_blocks.size() : 1));
     p->nudf = (int)udf_blocks.size();
     p->udf_wl = 0;
@@ -2218,7 +2145,7 @@ int ugks_step_plan_destroy(ugks_step_plan *p) {
     if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     void *ptrs[] = {p->d_blocks, p->d_face_off, p->d_cell_off, p->d_all_off, p->d_tile_off, p->d_cmom, p->d_qnext, p->d_walls, p->d_ghosts,
                     p->d_state, p->d_case_first, p->d_maxbits, p->d_max_dt, p->d_fsum, p->d_fstate, p->d_frec,
-                    p->d_tmap, p->d_udf_blocks};
+                    p->d_udf_blocks};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
     delete p;
@@ -2575,7 +2502,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
                  o_fsum = carve(sizeof(double) * kFSof(precision) * (size_t)P.nfaces, sizeof(double) * 16 * (size_t)P.nfaces),
                  o_qnext = carve(sizeof(d2) * (size_t)P.ncells, 0),
                  o_fstate = region(sizeof(double) * kFT * (size_t)P.nfaces),
-                 o_frec = region(sizeof(FaceRec) * (size_t)P.nfaces), o_tmap = region(sizeof(int) * (size_t)P.nfaces);
+                 o_frec = carve(sizeof(FaceRec) * (size_t)P.nfaces, sizeof(FaceRec) * (size_t)P.nfaces + ((sizeof(int) * (size_t)P.nfaces + 255) & ~(size_t)255));
     if (std::max(at, counted) > kNoAllocBytes) {
         char msg[200];
         snprintf(msg, sizeof msg, "step noalloc: the case needs %zu bytes of working memory; the allocation-free "
@@ -2601,7 +2528,6 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     P.d_fsum = (double *)(base + o_fsum);
     P.d_fstate = (double *)(base + o_fstate);
     P.d_frec = (FaceRec *)(base + o_frec);
-    P.d_tmap = (int *)(base + o_tmap);
     for (int b = 0; b < nblocks; b++) {
         host[b].cmom = P.d_cmom + T.off[2][b];
         host[b].qnext = (d2 *)(base + o_qnext) + T.off[1][b];
