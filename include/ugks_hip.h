@@ -210,15 +210,17 @@ int ugks_edgeConstGrad(ugks_block *blk, void *stream, void *Fin, int32_t this_fa
 
 /* ---- fused, batched step (layer 2) -------------------------------------- */
 /* One plan steps any number of blocks (of one or many independent cases) in
- * eight launches per step with the time step kept on the device.  It replaces
+ * five or six launches per step with the time step kept on the device.  It replaces
  * the sequence UGKSim.one_step drives per block (ugks_sim.py:407-501:
  * UGKS_flux, UGKS_update, calcTimeStep/updateTimeStep, updateAllBC) and
  * produces the same f, macro, Q, flux_macro, wall_cover and wall_fluxes.
  * Blocks given to one plan share one time step (ugks_sim.py:296-308);
  * independent cases that need their own time steps get their own plans. */
 enum { UGKS_FP64 = 0, UGKS_MIXED = 1 };
-/* launches per step, in order: face moments, face state, face flux, wall
- * faces, cell update, cell time step, time-step finalise, ghost cells */
+/* the parts of a step that ugks_step_run_timed launches and times one by one, in
+ * order: face moments, face state, face flux, wall faces, cell update, cell
+ * time step, time-step finalise, ghost cells.  A run puts the states and walls,
+ * and the last three, in one launch each. */
 #define UGKS_STEP_NKERNELS 8
 
 /* Device buffers of one block, in the layouts of layer 1.  f, flux_f_S,

@@ -1,29 +1,29 @@
 // ugks_fused.hip -- the batched, fused UGKS time step for gfx950.
 //
-// One step of every block of every case in eight launches, with no host
-// round trip (the reference issues ~30 launches per block per step plus two
-// blocking readbacks, ugks_block.py:1049-1329, :1415-1433):
+// One step of every block of every case in five launches (six with thousands
+// of wall faces), with no host round trip (the reference issues ~30 launches per
+// block per step plus two blocking readbacks, ugks_block.py:1049-1329,
+// :1415-1433):
 //
 //   k_faceA   one wavefront per interior face (S and W faces of all blocks):
 //             reconstruction (iFace) and the raw velocity moments of the face
 //             values (getFaceCons and the sums calcFaceQ needs).
-//   k_faceS   one thread per interior face: primary variables, slopes and
-//             time slope (getPLR/initMacroFlux), face heat flux (calcFaceQ)
-//             and the equilibrium part of the macro flux, folded into the
-//             per-face constants of the flux pass.
+//   k_wallS   one workgroup per diffuse/adsorbing wall face: reconstruction,
+//             accommodatingWallDist or adsorbingWall_P1 + S/D_P2, wallFlux,
+//             wallMassEnergyFluxes; and one thread per interior face: primary
+//             variables, slopes and time slope (getPLR/initMacroFlux), face
+//             heat flux (calcFaceQ) and the equilibrium part of the macro flux,
+//             folded into the per-face constants of the flux pass.
 //   k_faceC   one wavefront per interior face: reconstruction again, macro
 //             flux (macroFlux) and the per-velocity flux (distFlux).
-//   k_wall    one workgroup per diffuse/adsorbing wall face: reconstruction,
-//             accommodatingWallDist or adsorbingWall_P1 + S/D_P2, wallFlux,
-//             wallMassEnergyFluxes.
 //   k_update  one wavefront per cell: updateMacro + UGKS_update, the cell's
 //             moments for the next step's left/right face states (getAL/getAR)
 //             and its heat flux for the next update (calcQ).
-//   k_dt      one thread per cell: clFindDT and the per-block maximum.
-//   k_dtfin   one workgroup: the global time step with the reference's growth
-//             limit (ugks_sim.py:285-311, applied as one_step does, :430-446).
-//   k_ghost   one wavefront per ghost cell: every BC of every block
-//             (updateBC, ugks_block.py:621-665).
+//   k_end     one thread per cell: clFindDT and the per-block maximum; the last
+//             of these workgroups: the global time step with the reference's
+//             growth limit (ugks_sim.py:285-311, applied as one_step does,
+//             :430-446); and one wavefront per ghost cell: every BC of every
+//             block (updateBC, ugks_block.py:621-665).
 //
 // Items of all blocks are laid out back to back; a wavefront finds its block
 // by bisection of a prefix table.  f is stored as T2 = (g, h) pairs of T
@@ -539,10 +539,8 @@ __device__ __forceinline__ FaceGeo face_geo_of(const FaceRec &r, const Consts &C
 }
 
 // rec[fid]: face fid (per block, in tiled order)
-__global__ void __launch_bounds__(kT) k_facerec(const FBlock *__restrict__ blocks, const long long *__restrict__ off,
-                                                int nb, long long nfaces, FaceRec *__restrict__ rec) {
-    const long long fid = (long long)blockIdx.x * kT + threadIdx.x;
-    if (fid >= nfaces) return;
+__device__ __forceinline__ void face_record(const FBlock *__restrict__ blocks, const long long *__restrict__ off, int nb, long long fid,
+                                            FaceRec *__restrict__ rec) {
     const int b = find_block(off, nb, fid);
     const FBlock &B = blocks[b];
     const long long loc = fid - off[b];
@@ -634,11 +632,9 @@ __device__ __forceinline__ d2 face_heat(const double *S, d2 n, double U, double 
 // equilibrium part of the macro flux and the face heat flux (from the raw
 // moments about the face velocity) -- getPLR, initMacroFlux, calcFaceQ
 template <typename T>
-__global__ void __launch_bounds__(kT) k_faceS(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
-                                              long long nfaces, const double *__restrict__ fsum,
-                                              double *__restrict__ fstate, const DtState *__restrict__ ds) {
-    const long long fid = (long long)blockIdx.x * kT + threadIdx.x;
-    if (fid >= nfaces) return;
+__device__ __forceinline__ void face_state(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs, long long fid,
+                                           const double *__restrict__ fsum, double *__restrict__ fstate,
+                                           const DtState *__restrict__ ds) {
     const FaceRec R = recs[fid];
     const FBlock &B = blocks[R.b];
     const Consts &C = B.c;
@@ -994,12 +990,11 @@ struct WallItem { int block, wall; long long start; };
 // Beyond 7 the spills grow and the pass is a negligible share of the step.
 template <int NPT> constexpr int kWallWaves = NPT <= 7 ? 3 : 1;
 template <typename T, int NPT>
-__global__ void __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWallWaves<NPT>))) k_wall(const FBlock *__restrict__ blocks, const WallItem *__restrict__ items,
-                                             int nitems, const DtState *__restrict__ ds) {
+__device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, const WallItem *__restrict__ items, int nitems,
+                                          long long item, const DtState *__restrict__ ds) {
     __shared__ double red[kWavesT][16];
     __shared__ P2<T> wd[NPT * kT];   // reflected distribution (clAdsorb.c:377) for the specular mirror lookup
     __shared__ double sc[8];
-    const long long item = blockIdx.x;
     const WallItem W = items[find_item(items, nitems, item)];
     const FBlock &B = blocks[W.block];
     const Consts &C = B.c;
@@ -1224,6 +1219,25 @@ __global__ void __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWallWa
     (void)sc;
 }
 
+// The wall faces and the state pass in one launch: neither fills the chip or
+// reads what the other writes, and both are chains of dependent loads and
+// scalar-like arithmetic.  The first nwalls workgroups take a wall face each
+// (the longer chain), the rest 256 interior faces each.  One after the
+// other / together, us: 7.1 + 7.8 / 8.9 on two blocks of 6 x 10 cells, 8.8 + 13.2
+// / 15.5 on 64^2, 27 + 54 / 66 on 2 x 2 blocks of 128^2 (FP64), and a launch less.
+template <typename T, int NPT>
+__global__ void __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(kWallWaves<NPT>)))
+k_wallS(const FBlock *__restrict__ blocks, const WallItem *__restrict__ items, int nitems, long long nwalls,
+        const FaceRec *__restrict__ recs, long long nfaces, const double *__restrict__ fsum, double *__restrict__ fstate,
+        const DtState *__restrict__ ds) {
+    if (blockIdx.x < nwalls) {
+        wall_face<T, NPT>(blocks, items, nitems, blockIdx.x, ds);
+    } else {
+        const long long fid = ((long long)blockIdx.x - nwalls) * kT + threadIdx.x;
+        if (fid < nfaces) face_state<T>(blocks, recs, fid, fsum, fstate, ds);
+    }
+}
+
 // ======================================================= cell moments ====
 // M = sum_v (g, e_x g, e_y g, (|e|^2 g + h) / 2) of one cell in the global
 // frame: the getAL/getAR moments of its faces after rotation into the face
@@ -1276,10 +1290,7 @@ __device__ __forceinline__ void store_moments(d4 *dst, const double (&m)[4], int
 }
 
 template <typename T>
-__global__ void __launch_bounds__(kT) k_cellmom(const FBlock *__restrict__ blocks, const long long *__restrict__ off,
-                                                int nb, long long nall) {
-    const long long item = xcd_remap(blockIdx.x, gridDim.x) * kWavesT + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (item >= nall) return;
+__device__ __forceinline__ void cell_refresh(const FBlock *__restrict__ blocks, const long long *__restrict__ off, int nb, long long item) {
     const int lane = threadIdx.x & 63;
     const int b = find_block(off, nb, item);
     const FBlock &B = blocks[b];
@@ -1432,9 +1443,10 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
 // ============================================================ k_dt =========
 __device__ __forceinline__ unsigned long long dbits(double x) { return (unsigned long long)__double_as_longlong(x); }
 
-__global__ void __launch_bounds__(kT) k_dt(const FBlock *__restrict__ blocks, const long long *__restrict__ off, int nb,
-                                           const DtState *__restrict__ ds, unsigned long long *maxbits) {
-    const long long t = (long long)blockIdx.x * kT + threadIdx.x;
+// cells t = 256 group ..: clFindDT and the per-block maximum (atomics, so that any workgroup of any XCD adds to it)
+__device__ __forceinline__ void cell_dt(const FBlock *__restrict__ blocks, const long long *__restrict__ off, int nb,
+                                        const DtState *__restrict__ ds, unsigned long long *maxbits, long long group) {
+    const long long t = group * kT + threadIdx.x;
     const long long total = off[nb];
     double val = 0.0;
     int b = -1;
@@ -1483,19 +1495,18 @@ __global__ void __launch_bounds__(kT) k_dt(const FBlock *__restrict__ blocks, co
 // the global time step of each case (UGKSBlock.getDT + UGKSim.updateTimeStep),
 // applied once at the end of the step and once more when the next step's flux
 // loop re-evaluates it (ugks_sim.py:430-441); time advances by the first
-// value.  One thread per case; the blocks of case c are first[c] .. first[c+1]-1.
-__global__ void k_dtfin(DtState *dss, unsigned long long *maxbits, double *max_dt, const int *first, int ncases) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncases) return;
+// value.  Case c; its blocks are first[c] .. first[c+1]-1.
+__device__ __forceinline__ void case_dt(DtState *dss, unsigned long long *maxbits, double *max_dt, const int *first, int c) {
     DtState *ds = dss + c;
     double M = __builtin_inf();
     for (int b = first[c]; b < first[c + 1]; b++) {
-        double mx = __longlong_as_double((long long)maxbits[b]);
+        // past this XCD's L2: other XCDs' atomics made the maximum
+        double mx = __longlong_as_double((long long)__hip_atomic_load(maxbits + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
         double md = ds->CFL / mx;
         if (ds->suggest_dt > 0.0 && ds->suggest_dt < md) md = ds->suggest_dt;
         max_dt[b] = md;
         M = fmin(M, md);
-        maxbits[b] = 0ull;
+        __hip_atomic_store(maxbits + b, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (ds->force_time) {       // dt held at the value that lands on max_time (ugks_sim.py:292, :673-675)
         ds->time += ds->dt;
@@ -1542,11 +1553,9 @@ __global__ void __launch_bounds__(kT) k_parabc(const FBlock *__restrict__ blocks
 
 // edge-exchange corner check (clGhostRoutines.c:491-512): a joined face whose
 // end vertices do not coincide with the partner face's (1e-6) has its ghost row
-// flipped, if its orientation flag asks for it.  Thread 4 b + k checks face k
-// of block b from the vertices as they stand, at every run call.
-__global__ void k_flipidx(FBlock *__restrict__ blocks, int nb) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= 4 * nb) return;
+// flipped, if its orientation flag asks for it.  t = 4 b + k checks face k of
+// block b from the vertices as they stand.
+__device__ __forceinline__ void join_corner(FBlock *blocks, int t) {
     FBlock &F = blocks[t >> 2];
     const int k = t & 3;
     int flip = 0;
@@ -1578,10 +1587,8 @@ __global__ void k_flipidx(FBlock *__restrict__ blocks, int nb) {
 struct GhostItem { int block, face; long long start; };
 
 template <typename T>
-__global__ void __launch_bounds__(kT) k_ghost(const FBlock *__restrict__ blocks, const GhostItem *__restrict__ items,
-                                              int nitems, long long nghosts) {
-    const long long item = (long long)blockIdx.x * kWavesT + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (item >= nghosts) return;
+__device__ __forceinline__ void ghost_cell(const FBlock *__restrict__ blocks, const GhostItem *__restrict__ items, int nitems,
+                                           long long item) {
     const int lane = threadIdx.x & 63;
     const GhostItem GI = items[find_item(items, nitems, item)];
     const FBlock &B = blocks[GI.block];
@@ -1704,7 +1711,7 @@ __global__ void __launch_bounds__(kT) k_ghost(const FBlock *__restrict__ blocks,
     } else {
         const int noi = (face == GNORTH || face == GEAST) ? gi : ei, noj = (face == GNORTH || face == GEAST) ? gj : ej;
         Q = B.Q[(size_t)(ei - C.G) * C.nj + (ej - C.G)];
-        pr = B.macro[(size_t)(ei - C.G) * C.nj + (ej - C.G)];
+        pr = B.macro_new[(size_t)(ei - C.G) * C.nj + (ej - C.G)];     // (macro is being written from it)
         d2 l = to_local(mk2(pr.s1, pr.s2), B.normal[((size_t)noi * C.NJ + noj) * 2 + (ns ? SOUTH : WEST)]);
         pr.s1 = l.x; pr.s2 = l.y;
         if (type == 6) { pr.s0 = wp.s0; pr.s3 = wp.s3; }
@@ -1715,6 +1722,78 @@ __global__ void __launch_bounds__(kT) k_ghost(const FBlock *__restrict__ blocks,
         put(v, P2<T>{(T)fe.x, (T)fe.y});
     }
     finish();
+}
+
+// What a run call derives again, in one launch: the moments of every cell, the
+// face records, and the join corners: those go into flipidx of the block
+// records, which nothing else here reads (so the records stay scalar loads).
+template <typename T>
+__global__ void __launch_bounds__(kT) k_refresh(const FBlock *__restrict__ blocks, FBlock *joins, int nb, const long long *__restrict__ all_off, long long nall,
+                                                long long cell_groups, const long long *__restrict__ face_off, long long nfaces,
+                                                long long face_groups, FaceRec *__restrict__ rec) {
+    const long long g = blockIdx.x;
+    if (g < cell_groups) {
+        const long long item = xcd_remap(g, cell_groups) * kWavesT + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (item < nall) cell_refresh<T>(blocks, all_off, nb, item);
+    } else if (g < cell_groups + face_groups) {
+        const long long fid = (g - cell_groups) * kT + threadIdx.x;
+        if (fid < nfaces) face_record(blocks, face_off, nb, fid, rec);
+    } else {
+        const int t = (int)(g - cell_groups - face_groups) * kT + threadIdx.x;
+        if (t < 4 * nb) join_corner(joins, t);
+    }
+}
+
+// The end of a step in one launch: the ghost cells (which read the new state
+// the update left in macro_new), the cells' time steps, and the global ones by
+// whichever time-step workgroup finishes last (ticket; it waits for nobody).
+// As three launches, one after the other / together, us: 5.0 + 4.4 + 1.9 / 7.4 on
+// two blocks of 6 x 10 cells, 7.3 + 4.8 + 4.5 / 7.7 on 64^2, 42 + 18 + 6 / 52 on
+// 2 x 2 blocks of 128^2 (FP64), and two launches less.
+struct EndOfStep {
+    const GhostItem *ghosts;
+    int nghost_items;
+    long long nghosts, nghost_groups, ndt_groups;
+    const long long *cell_off;
+    int nb, ncases;
+    DtState *ds;
+    unsigned long long *maxbits;
+    double *max_dt;
+    const int *case_first;
+    unsigned *ticket;          // 0 between launches
+};
+template <typename T>
+__global__ void __launch_bounds__(kT) k_end(const FBlock *__restrict__ blocks, EndOfStep e) {
+    const long long g = blockIdx.x;
+    if (g >= e.ndt_groups) {
+        const long long item = (g - e.ndt_groups) * kWavesT + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        if (item < e.nghosts) ghost_cell<T>(blocks, e.ghosts, e.nghost_items, item);
+        return;
+    }
+    __shared__ int last;
+    cell_dt(blocks, e.cell_off, e.nb, e.ds, e.maxbits, g);
+    // Only the maxima cross workgroups, and those are atomics at the device's
+    // scope on both sides: it is enough that a wavefront's are performed before
+    // its workgroup draws a ticket.  A __threadfence() here would also write the
+    // L2 back per workgroup (16 blocks of 128^2: 195 us instead of 138 for the
+    // three launches).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) last = atomicAdd(e.ticket, 1u) == (unsigned)(e.ndt_groups - 1);
+    __syncthreads();
+    if (!last) return;
+    for (int c = threadIdx.x; c < e.ncases; c += kT) case_dt(e.ds, e.maxbits, e.max_dt, e.case_first, c);
+    if (threadIdx.x == 0) __hip_atomic_store(e.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// the same work in launches of its own, for per-kernel timing
+__global__ void __launch_bounds__(kT) k_dt(const FBlock *__restrict__ blocks, const long long *__restrict__ off, int nb,
+                                           const DtState *__restrict__ ds, unsigned long long *maxbits) {
+    cell_dt(blocks, off, nb, ds, maxbits, blockIdx.x);
+}
+__global__ void k_dtfin(DtState *dss, unsigned long long *maxbits, double *max_dt, const int *first, int ncases) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < ncases) case_dt(dss, maxbits, max_dt, first, c);
 }
 
 // FP64 -> FP32 conversion of f (the mixed-precision state starts from the FP64 initial state)
@@ -1763,6 +1842,7 @@ struct ugks_step_plan {
     hipGraphExec_t graph_exec;
     unsigned long long *d_maxbits;
     double *d_max_dt;
+    unsigned *d_ticket;                 // 0 between steps (k_end)
     std::vector<FBlock> host_blocks;
 };
 
@@ -1801,10 +1881,24 @@ template <typename T> void faceC(ugks_step_plan *p, hipStream_t s, int fw) {
     if (fw == 1) faceC_m<T, 1>(p, s); else if (fw == 2) faceC_m<T, 2>(p, s); else faceC_m<T, 4>(p, s);
 }
 
-// ev != nullptr: record ev[0..kLaunches] around the launches (per-kernel timing)
+// ev != nullptr: per-kernel timing, with ev[0..kLaunches] recorded around
+// launches of their own for the parts that a step otherwise runs together
 constexpr int kLaunches = UGKS_STEP_NKERNELS;
+template <typename T, int NPT> void launch_wallS(ugks_step_plan *p, hipStream_t s, long long nwalls, long long nfaces) {
+    const long long groups = nwalls + (nfaces + kT - 1) / kT;
+    if (groups > 0)
+        hipLaunchKernelGGL((k_wallS<T, NPT>), dim3((unsigned)groups), dim3(kT), 0, s, p->d_blocks, (const WallItem *)p->d_walls,
+                           p->nwall_items, nwalls, (const FaceRec *)p->d_frec, nfaces, (const double *)p->d_fsum, p->d_fstate,
+                           (const DtState *)p->d_state);
+}
+template <typename T> void launch_end(ugks_step_plan *p, hipStream_t s, bool dt) {
+    const long long ghost_groups = (p->nghosts + kWavesT - 1) / kWavesT, dt_groups = dt ? (p->ncells + kT - 1) / kT : 0;
+    const EndOfStep e{p->d_ghosts, p->nghost_items, p->nghosts, ghost_groups, dt_groups, p->d_cell_off, p->nb, p->ncases, p->d_state,
+                      p->d_maxbits, p->d_max_dt, p->d_case_first, p->d_ticket};
+    if (ghost_groups + dt_groups > 0)
+        hipLaunchKernelGGL((k_end<T>), dim3((unsigned)(ghost_groups + dt_groups)), dim3(kT), 0, s, (const FBlock *)p->d_blocks, e);
+}
 template <typename T, int NPT> int launch_step(ugks_step_plan *p, hipStream_t s, hipEvent_t *ev) {
-    const unsigned gt = (unsigned)((p->nfaces + kT - 1) / kT);             // one thread per face
     if (p->nudf > 0)
         hipLaunchKernelGGL(k_parabc, dim3((unsigned)p->nudf, (unsigned)((p->udf_wl + kT - 1) / kT)), dim3(kT), 0, s,
                            p->d_blocks, (const int *)p->d_udf_blocks, (const DtState *)p->d_state);
@@ -1812,42 +1906,42 @@ template <typename T, int NPT> int launch_step(ugks_step_plan *p, hipStream_t s,
     if (p->nfaces > 0)
         faceA<T>(p, s, p->fa_waves);
     if (ev) (void)hipEventRecord(ev[1], s);
-    if (p->nfaces > 0)
-        hipLaunchKernelGGL((k_faceS<T>), dim3(gt), dim3(kT), 0, s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
-                           (const double *)p->d_fsum, p->d_fstate, (const DtState *)p->d_state);
+    // Walls beside the states while they are few enough to be latency, not work:
+    // 9 us off a mixed step of 2 x 2 blocks of 128^2 (1,028 workgroups).  With 16 blocks of 128^2 (10,256) the launches take as long together
+    // as apart, and an update straight behind the flux pass takes longer than
+    // one behind the walls: 6.00 against 5.96 ms a step.
+    const bool beside = !ev && p->nwalls + (p->nfaces + kT - 1) / kT <= 4096;
+    launch_wallS<T, NPT>(p, s, beside ? p->nwalls : 0, p->nfaces);
     if (ev) (void)hipEventRecord(ev[2], s);
     if (p->nfaces > 0)
         faceC<T>(p, s, p->fc_waves);
     if (ev) (void)hipEventRecord(ev[3], s);
-    if (p->nwalls > 0)
-        hipLaunchKernelGGL((k_wall<T, NPT>), dim3((unsigned)p->nwalls), dim3(kT), 0, s, p->d_blocks, p->d_walls,
-                           p->nwall_items, p->d_state);
+    if (!beside) launch_wallS<T, NPT>(p, s, p->nwalls, 0);
     if (ev) (void)hipEventRecord(ev[4], s);
     hipLaunchKernelGGL((k_update<T>), dim3((unsigned)p->ntiles), dim3(kT), 0, s, p->d_blocks, p->d_tile_off, p->nb,
                        p->ntiles, p->d_state);
-    if (ev) (void)hipEventRecord(ev[5], s);
-    hipLaunchKernelGGL(k_dt, dim3((unsigned)((p->ncells + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks, p->d_cell_off,
-                       p->nb, p->d_state, p->d_maxbits);
-    if (ev) (void)hipEventRecord(ev[6], s);
-    hipLaunchKernelGGL(k_dtfin, dim3((unsigned)((p->ncases + 63) / 64)), dim3(64), 0, s, p->d_state, p->d_maxbits,
-                       p->d_max_dt, (const int *)p->d_case_first, p->ncases);
-    if (ev) (void)hipEventRecord(ev[7], s);
-    if (p->nghosts > 0)
-        hipLaunchKernelGGL((k_ghost<T>), dim3((unsigned)((p->nghosts + kWavesT - 1) / kWavesT)), dim3(kT), 0, s,
-                           p->d_blocks, p->d_ghosts, p->nghost_items, p->nghosts);
+    if (ev) {
+        (void)hipEventRecord(ev[5], s);
+        hipLaunchKernelGGL(k_dt, dim3((unsigned)((p->ncells + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks, p->d_cell_off,
+                           p->nb, p->d_state, p->d_maxbits);
+        (void)hipEventRecord(ev[6], s);
+        hipLaunchKernelGGL(k_dtfin, dim3((unsigned)((p->ncases + 63) / 64)), dim3(64), 0, s, p->d_state, p->d_maxbits,
+                           p->d_max_dt, (const int *)p->d_case_first, p->ncases);
+        (void)hipEventRecord(ev[7], s);
+    }
+    launch_end<T>(p, s, !ev);
     if (ev) (void)hipEventRecord(ev[8], s);
     return ugks_rt::check_launch("ugks_step_run");
 }
 
-// moments of every cell from f as it stands (f may have been changed between
-// runs), and the face records from the geometry as it stands
+// at every run call: moments of every cell from f as it stands (f may have
+// been changed between runs), and the face records and join corners from the
+// geometry as it stands
 template <typename T> int refresh_moments(ugks_step_plan *p, hipStream_t s) {
-    hipLaunchKernelGGL((k_cellmom<T>), dim3((unsigned)((p->nall + kWavesT - 1) / kWavesT)), dim3(kT), 0, s, p->d_blocks,
-                       p->d_all_off, p->nb, p->nall);
-    if (p->nfaces > 0)
-        hipLaunchKernelGGL(k_facerec, dim3((unsigned)((p->nfaces + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks,
-                           p->d_face_off, p->nb, p->nfaces, p->d_frec);
-    hipLaunchKernelGGL(k_flipidx, dim3((unsigned)((4 * p->nb + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks, p->nb);
+    const long long cells = (p->nall + kWavesT - 1) / kWavesT, faces = (p->nfaces + kT - 1) / kT, corners = (4 * p->nb + kT - 1) / kT;
+    hipLaunchKernelGGL((k_refresh<T>), dim3((unsigned)(cells + faces + corners)), dim3(kT), 0, s,
+                       (const FBlock *)p->d_blocks, p->d_blocks, p->nb, (const long long *)p->d_all_off, p->nall, cells, (const long long *)p->d_face_off, p->nfaces, faces,
+                       p->d_frec);
     return ugks_rt::check_launch("ugks_step: cell moments, face records and join corners");
 }
 int refresh(ugks_step_plan *p, hipStream_t s) {
@@ -1900,9 +1994,7 @@ template <typename T> int autotune(ugks_step_plan *p, hipStream_t s, int reps, i
             const int fw = cand[c];
             // kC reads kA's results through kS: run the chain once, then time the kernel alone
             faceA<T>(p, s, which == 0 ? fw : p->fa_waves);
-            hipLaunchKernelGGL((k_faceS<T>), dim3((unsigned)((p->nfaces + kT - 1) / kT)), dim3(kT), 0, s, p->d_blocks,
-                               (const FaceRec *)p->d_frec, p->nfaces, (const double *)p->d_fsum, p->d_fstate,
-                               (const DtState *)p->d_state);
+            launch_wallS<T, 1>(p, s, 0, p->nfaces);
             (void)hipEventRecord(e0, s);
             for (int r = 0; r < reps; r++) {
                 if (which == 0) faceA<T>(p, s, fw);
@@ -2087,6 +2179,7 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     (void)alloc((void **)&p->d_case_first, sizeof(int) * (ncases + 1));
     (void)alloc((void **)&p->d_maxbits, sizeof(unsigned long long) * nblocks);
     (void)alloc((void **)&p->d_max_dt, sizeof(double) * nblocks);
+    (void)alloc((void **)&p->d_ticket, sizeof(unsigned));
     (void)alloc((void **)&p->d_fsum, sizeof(double) * kFSof(precision) * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_fstate, sizeof(double) * kFT * (size_t)p->nfaces);
     (void)alloc((void **)&p->d_frec, sizeof(FaceRec) * (size_t)p->nfaces);
@@ -2121,6 +2214,7 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
     if (e == hipSuccess)
         e = hipMemcpy(p->d_case_first, case_first.data(), sizeof(int) * (ncases + 1), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(p->d_maxbits, zeros.data(), sizeof(unsigned long long) * nblocks, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(p->d_ticket, zeros.data(), sizeof(unsigned), hipMemcpyHostToDevice);
     std::vector<double> md0(nblocks);
     for (int b = 0; b < nblocks; b++) md0[b] = dtd[case_of_block ? case_of_block[b] : 0].max_dt;
     if (e == hipSuccess) e = hipMemcpy(p->d_max_dt, md0.data(), sizeof(double) * nblocks, hipMemcpyHostToDevice);
@@ -2144,7 +2238,7 @@ int ugks_step_plan_destroy(ugks_step_plan *p) {
     if (p->graph) (void)hipGraphDestroy(p->graph);
     if (p->cap_stream) (void)hipStreamDestroy(p->cap_stream);
     void *ptrs[] = {p->d_blocks, p->d_face_off, p->d_cell_off, p->d_all_off, p->d_tile_off, p->d_cmom, p->d_qnext, p->d_walls, p->d_ghosts,
-                    p->d_state, p->d_case_first, p->d_maxbits, p->d_max_dt, p->d_fsum, p->d_fstate, p->d_frec,
+                    p->d_state, p->d_case_first, p->d_maxbits, p->d_max_dt, p->d_ticket, p->d_fsum, p->d_fstate, p->d_frec,
                     p->d_udf_blocks};
     for (void *q : ptrs)
         if (q) (void)hipFree(q);
@@ -2353,26 +2447,23 @@ struct NoAllocTables {
     int udf[kNoAllocMaxBlocks];
     int nb, nwall, nghost, nudf;
 };
-static_assert(sizeof(NoAllocTables) < 4000, "the tables travel as a kernel argument");
+static_assert(sizeof(NoAllocTables) < 3900, "the tables travel as a kernel argument");
 
 __global__ void k_put_block(FBlock F, FBlock *dst) {
     if (threadIdx.x == 0) *dst = F;
 }
 __global__ void k_put_tables(NoAllocTables T, long long *off, WallItem *walls, GhostItem *ghosts, int *udf,
-                             int *case_first) {
+                             int *case_first, const ugks_dt_desc *in, DtState *ds, double *max_dt, unsigned long long *maxbits) {
     const int t = threadIdx.x;
     if (t < T.nb + 1)
         for (int k = 0; k < 4; k++) off[k * (T.nb + 1) + t] = T.off[k][t];
     if (t < T.nwall) walls[t] = T.walls[t];
     if (t < T.nghost) ghosts[t] = T.ghosts[t];
     if (t < T.nudf) udf[t] = T.udf[t];
-    if (t == 0) { case_first[0] = 0; case_first[1] = T.nb; }
-}
-// the case's time-step state from the caller's descriptor (device memory), and
-// the per-block time-step words cleared (the last call left its own there)
-__global__ void k_dt_in(const ugks_dt_desc *in, DtState *ds, double *max_dt, unsigned long long *maxbits, int nb) {
-    const int t = threadIdx.x;
-    if (t < nb) { max_dt[t] = in->max_dt; maxbits[t] = 0ull; }
+    if (t == 0) { case_first[0] = 0; case_first[1] = T.nb; case_first[2] = 0; }      // (and the ticket)
+    // the case's time-step state from the caller's descriptor (device memory), and
+    // the per-block time-step words cleared (the last call left its own there)
+    if (t < T.nb) { max_dt[t] = in->max_dt; maxbits[t] = 0ull; }
     if (t == 0) {
         DtState d{in->dt, in->dt, in->dt, in->time, in->CFL, in->delta_dt, in->suggest_dt, in->Kn_eff,
                   in->step, 0, in->force_time, 0};
@@ -2496,7 +2587,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     auto region = [&](size_t bytes) { return carve(bytes, bytes); };
     const size_t o_blocks = region(sizeof(FBlock) * nblocks), o_off = region(sizeof(long long) * 4 * (nblocks + 1)),
                  o_walls = region(sizeof(WallItem) * 4 * nblocks), o_ghosts = region(sizeof(GhostItem) * 4 * nblocks),
-                 o_udf = region(sizeof(int) * nblocks), o_case = region(sizeof(int) * 2), o_state = region(sizeof(DtState)),
+                 o_udf = region(sizeof(int) * nblocks), o_case = region(sizeof(int) * 3), o_state = region(sizeof(DtState)),
                  o_maxbits = region(sizeof(unsigned long long) * nblocks), o_maxdt = region(sizeof(double) * nblocks),
                  o_cmom = region(sizeof(d4) * (size_t)P.nall),
                  o_fsum = carve(sizeof(double) * kFSof(precision) * (size_t)P.nfaces, sizeof(double) * 16 * (size_t)P.nfaces),
@@ -2521,6 +2612,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     P.d_ghosts = (GhostItem *)(base + o_ghosts);
     P.d_udf_blocks = (int *)(base + o_udf);
     P.d_case_first = (int *)(base + o_case);
+    P.d_ticket = (unsigned *)(P.d_case_first + 2);
     P.d_state = (DtState *)(base + o_state);
     P.d_maxbits = (unsigned long long *)(base + o_maxbits);
     P.d_max_dt = (double *)(base + o_maxdt);
@@ -2534,9 +2626,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
         hipLaunchKernelGGL(k_put_block, dim3(1), dim3(64), 0, s, host[b], P.d_blocks + b);
     }
     hipLaunchKernelGGL(k_put_tables, dim3(1), dim3(kT), 0, s, T, off, P.d_walls, P.d_ghosts, P.d_udf_blocks,
-                       P.d_case_first);
-    hipLaunchKernelGGL(k_dt_in, dim3(1), dim3(64), 0, s, (const ugks_dt_desc *)dt, P.d_state, P.d_max_dt, P.d_maxbits,
-                       nblocks);
+                       P.d_case_first, (const ugks_dt_desc *)dt, P.d_state, P.d_max_dt, P.d_maxbits);
     int rc = ugks_rt::check_launch("step noalloc: set-up");
     if (!rc) rc = refresh(&P, s);
     for (int k = 0; k < nsteps && !rc; k++)

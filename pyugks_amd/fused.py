@@ -4,8 +4,8 @@
 simulations (cases), that the reference-shaped path has initialised
 (geometry, initial f, ghosts, first time step; the sequence of
 ugks_sim.py:52-92) and advances all of their blocks together: each step is
-eight launches over every block of every case, with each case's time step
-kept on the device (one UGKSim.one_step per case, ugks_sim.py:407-501).
+five launches over every block of every case (six with thousands of wall
+faces), with each case's time step kept on the device (one UGKSim.one_step per case, ugks_sim.py:407-501).
 With ``graph=True`` the step runs as replays of a captured HIP graph.  With
 ``precision="mixed"`` f and the per-velocity face fluxes are stored and
 computed in FP32; moments, the macroscopic update, heat fluxes, equilibrium
