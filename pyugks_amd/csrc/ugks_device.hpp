@@ -164,9 +164,9 @@ __device__ __forceinline__ d2 to_local(d2 in, d2 n) {
 }
 
 // relaxTime (clFunctions.c:8-32)
-__device__ __forceinline__ double relax_time(const Consts &C, d4 p) {
-    double base = (C.Kn / p.s0);
-    double pw = pow(p.s3, 1.0 - C.omega);
+// base = Kn / rho
+__device__ __forceinline__ double relax_time_of(const Consts &C, double base, double lam) {
+    double pw = pow(lam, 1.0 - C.omega);
     switch (C.relax) {
     case 0: return base * 0.79788456080286541 * pw;
     case 1: return (5. / 8.) * base * sqrt(kPi) * pw;
@@ -174,6 +174,7 @@ __device__ __forceinline__ double relax_time(const Consts &C, d4 p) {
     default: return base * pw;
     }
 }
+__device__ __forceinline__ double relax_time(const Consts &C, d4 p) { return relax_time_of(C, C.Kn / p.s0, p.s3); }
 
 // fM (clFunctions.c:49-58): weighted Maxwellian (g, h)
 __device__ __forceinline__ d2 maxwell(const Consts &C, d4 p, d2 uv, int v) {

@@ -256,12 +256,11 @@ inline bool stencil_span_fits(long long NJ, long long NV, int method, int precis
 }
 template <typename T> using V2 = T __attribute__((ext_vector_type(2)));
 // a store that is not read again soon (per-velocity fluxes, the new f): it
-// streams past the caches instead of evicting stencil data still in use
+// streams past the caches instead of evicting stencil data still in use.
 template <typename T> __device__ __forceinline__ void stream_store(V2<T> *p, V2<T> x) { __builtin_nontemporal_store(x, p); }
 template <typename T> __device__ __forceinline__ void stream_store(__attribute__((address_space(1))) V2<T> *p, V2<T> x) {
     __builtin_nontemporal_store(x, p);
 }
-
 // element v of a wavefront-uniform row: the row stays a scalar base and the lane adds a 32-bit byte offset
 template <typename T> __device__ __forceinline__ AS1 V2<T> *vslot(AS1 V2<T> *row, int v) {
     return (AS1 V2<T> *)((AS1 char *)row + (unsigned)v * (unsigned)sizeof(V2<T>));
@@ -280,6 +279,12 @@ __device__ __forceinline__ double weight_at(const Consts &C, int v) {
 __device__ __forceinline__ double uniform_d(double x) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(x);
     const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// lane k's double, held in scalar registers
+template <int K> __device__ __forceinline__ double lane_d(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, K), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), K);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 // the reciprocals go through an empty asm so the compiler cannot turn the
@@ -1328,27 +1333,62 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const int b = find_block(off, nb, tile);
     const FBlock &B = blocks[b];
     const Consts &C = B.c;
-    const long long t = tile - off[b];
-    const int nrp = (C.nj + 1) >> 1;
+    const unsigned t = (unsigned)(tile - off[b]), nrp = (unsigned)(C.nj + 1) >> 1;
     const int mi = 2 * (int)(t / nrp) + (wv >> 1), mj = 2 * (int)(t % nrp) + (wv & 1);
     if (mi >= C.ni || mj >= C.nj) return;
     const long long cell = (long long)mi * C.nj + mj;
     const int gi = mi + C.G, gj = mj + C.G;
     const size_t c0 = (size_t)gi * C.NJ + gj;
     const double dt = ds[B.cs].dt_up;
-    // updateMacro (clUGKS.c:1158-1187)
+    // updateMacro (clUGKS.c:1158-1187) and the constants of UGKS_update
+    // (:1189-1257).  All of it is the same for the wavefront's 64 lanes, and
+    // most of it is divisions and a power: those that do not wait for one
+    // another are taken by different lanes of one division (7 instead of 24, one
+    // pow instead of two).  Evaluated by every lane alike it was 900 VALU
+    // instructions, as many as 6 turns of the velocity loop (9 turns on 24^2
+    // velocities, 18 on 33^2), and 9 registers more: the mixed update of 16
+    // blocks of 128^2 went from 1.61 to 1.55 ms with it, that of 64^2 from 28.2 to
+    // 26.7 us; the FP64 one, bound by its bytes, stayed as it was.
+    // Each operation rounds by itself (contraction off), but for the FMAs that
+    // the conserved state takes the flux difference in.
+    const double A = B.area[c0], gm1 = C.gam - 1.0;
     const d4 pold = B.macro[cell];
-    const double A = B.area[c0];
-    const d4 dW = ((B.fmS[c0] - B.fmS[c0 + 1]) + B.fmW[c0]) - B.fmW[c0 + C.NJ];
-    const d4 p = to_primary(C, to_conserved(C, pold) + dW / A);
     const d2 Q = B.qnext[cell];
+    const int part = lane & 7;
+    d4 p;
+    double rl, tau2, r1, r3;
+    {
+#pragma clang fp contract(off)
+        // dW / A of component k in lane k, 0.5 rho / lambda in 4, 1 / A in 5, 1 / K in 6
+        const int k = lane & 3;
+        const double dW = ((((const double *)(B.fmS + c0))[k] - ((const double *)(B.fmS + c0 + 1))[k]) +
+                           ((const double *)(B.fmW + c0))[k]) - ((const double *)(B.fmW + c0 + C.NJ))[k];
+        r1 = (part < 4 ? dW : part == 4 ? 0.5 * pold.s0 : 1.0) / (part < 4 || part == 5 ? A : part == 4 ? pold.s3 : C.K);
+        const double w0 = pold.s0 + lane_d<0>(r1);
+        const double w1 = fma(pold.s0, pold.s1, lane_d<1>(r1)), w2 = fma(pold.s0, pold.s2, lane_d<2>(r1));
+        // u, v, 0.5 (w1^2 + w2^2) / rho; 0.5 rho / (gamma - 1) and the old state's 0.5 rho / lambda / (gamma - 1)
+        const double r2 = (part == 0 ? w1 : part == 1 ? w2 : part == 2 ? 0.5 * fma(w1, w1, w2 * w2)
+                           : part == 3 ? 0.5 * w0 : lane_d<4>(r1)) / (part < 3 ? w0 : gm1);
+        const double e0 = fma(0.5 * pold.s0, fma(pold.s1, pold.s1, pold.s2 * pold.s2), lane_d<4>(r2));
+        const double w3 = e0 + lane_d<3>(r1);
+        p.s0 = w0;
+        p.s1 = lane_d<0>(r2);
+        p.s2 = lane_d<1>(r2);
+        p.s3 = lane_d<3>(r2) / (w3 - lane_d<2>(r2));
+        // even lanes the old state, odd lanes the new one
+        const bool odd = lane & 1;
+        const double rho = odd ? p.s0 : pold.s0, lam = odd ? p.s3 : pold.s3;
+        const int q = part >> 1;
+        r3 = (q == 0 ? C.Kn : q == 1 ? lam : q == 2 ? 0.8 * (1 - C.Pr) * (lam * lam) : C.K) /
+             (q == 1 ? kPi : q == 3 ? 2.0 * lam : rho);
+        tau2 = relax_time_of(C, odd ? lane_d<1>(r3) : lane_d<0>(r3), lam);
+        rl = rho * (odd ? lane_d<3>(r3) : lane_d<2>(r3));
+    }
     if (lane == 0) {
         B.macro_new[cell] = p;
         B.residual[cell] = pold;
         B.Q[cell] = Q;
     }
-    // UGKS_update (clUGKS.c:1189-1257)
-    const double tau_old = relax_time(C, pold), tau = relax_time(C, p);
     const bool sep = C.nut > 0;
     double (*tab)[64] = tabs[wv];
     if (sep) {
@@ -1363,26 +1403,22 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const double rlo = pold.s0 * (pold.s3 / kPi), rln = p.s0 * (p.s3 / kPi);
-    const double so = 0.8 * (1 - C.Pr) * (pold.s3 * pold.s3) / pold.s0, sn = 0.8 * (1 - C.Pr) * (p.s3 * p.s3) / p.s0;
-    const double hfo = C.K / (2.0 * pold.s3), hfn = C.K / (2.0 * p.s3);
-    const double rA = 1.0 / A, rden = 1.0 / (1.0 + 0.5 * dt / tau);
-    const double htn = (0.5 * dt) / tau, hto = (0.5 * dt) / tau_old;
-    // the per-cell constants of the velocity loop in scalar registers: the FP32
-    // update then needs 74 VGPRs (six waves per SIMD) instead of 104, the FP64 one 84
-    // (five); held to 72 for seven waves, the FP32 one spills and runs slower
+    // the per-cell constants of the velocity loop in scalar registers, and one
+    // 32-bit lane offset for the five rows: 71 VGPRs (seven waves per SIMD) in
+    // mixed mode, 81 in FP64 (five; held to 80 for six, 2 x 2 blocks of 128^2 took
+    // 969 us instead of 963, the channel 6.05 ms instead of 5.98)
     const double po1 = uniform_d(pold.s1), po2 = uniform_d(pold.s2), po3 = uniform_d(pold.s3);
-    const double pn1 = uniform_d(p.s1), pn2 = uniform_d(p.s2), pn3 = uniform_d(p.s3);
+    const double pn1 = p.s1, pn2 = p.s2, pn3 = uniform_d(p.s3);
     const double Qx = uniform_d(Q.x), Qy = uniform_d(Q.y);
-    const double urlo = uniform_d(rlo), urln = uniform_d(rln), uso = uniform_d(so), usn = uniform_d(sn);
-    const double uhfo = uniform_d(hfo), uhfn = uniform_d(hfn), urA = uniform_d(rA), urden = uniform_d(rden);
-    const double uhtn = uniform_d(htn), uhto = uniform_d(hto), urK = uniform_d(1.0 / C.K);
+    const double ht = (0.5 * dt) / tau2;
+    const double uhto = lane_d<0>(ht), uhtn = lane_d<1>(ht), urden = uniform_d(1.0 / (1.0 + uhtn));
+    const double urlo = lane_d<0>(rl), urln = lane_d<1>(rl), uso = lane_d<4>(r3), usn = lane_d<5>(r3);
+    const double uhfo = lane_d<6>(r3), uhfn = lane_d<7>(r3), urA = lane_d<5>(r1), urK = lane_d<6>(r1);
     // this cell's velocities in f and in the four face fluxes: uniform bases, 32-bit lane offsets
     const long long NV = C.NV;
     AS1 V2<T> *fc = (AS1 V2<T> *)B.f + c0 * NV;
-    const AS1 V2<T> *fS = (const AS1 V2<T> *)B.fluxS + c0 * NV;
-    const AS1 V2<T> *fW = (const AS1 V2<T> *)B.fluxW + c0 * NV;
-    const unsigned nS = (unsigned)NV, nE = (unsigned)(C.NJ * NV);
+    AS1 V2<T> *fS = (AS1 V2<T> *)B.fluxS + c0 * NV, *fN = fS + NV;
+    AS1 V2<T> *fW = (AS1 V2<T> *)B.fluxW + c0 * NV, *fE = fW + (long long)C.NJ * NV;
     // tensor indices of v = lane + 64 k, advanced without integer division
     int iu = 0, jv = 0, diu = 0, djv = 0;
     // the grid width in a register: the flux stores could alias the block
@@ -1397,7 +1433,7 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     d2 enext = lane < C.NV ? quad_at(C, lane) : d2{0.0, 0.0};
     double wnext = lane < C.NV ? weight_at(C, lane) : 0.0;
     for (int v = lane; v < C.NV; v += 64) {
-        const V2<T> fo = fc[v], sS = fS[v], nS_ = fS[v + nS], wW = fW[v], eW = fW[v + nE];
+        const V2<T> fo = *vslot<T>(fc, v), sS = *vslot<T>(fS, v), nS_ = *vslot<T>(fN, v), wW = *vslot<T>(fW, v), eW = *vslot<T>(fE, v);
         const d2 e = enext;
         const double w = wnext;
         {   // the next velocity's table entries (this one's again on the last round: no branch)
@@ -1430,7 +1466,7 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
         const double nh = (fh + flh + (uhtn * feqNh + uhto * (feqOh - fh))) * urden;
         const T tg = (T)ng, th = (T)nh;
         if (isnan(tg) || isnan(th)) nan_seen = true;
-        stream_store<T>(fc + v, V2<T>{tg, th});
+        stream_store<T>(vslot<T>(fc, v), V2<T>{tg, th});
         // the new cell's moments and heat flux (the next step's getAL / getAR and update inputs)
         add_moments<T>(e, tg, th, mom);
         add_heat<T>(nx, ny, cn, urK, tg, th, heat);
