@@ -257,10 +257,17 @@ inline bool stencil_span_fits(long long NJ, long long NV, int method, int precis
 template <typename T> using V2 = T __attribute__((ext_vector_type(2)));
 // a store that is not read again soon (per-velocity fluxes, the new f): it
 // streams past the caches instead of evicting stencil data still in use.
+// KEEP: an ordinary store, for fluxes that stay in the 256 MB last-level cache
+// until the update reads them.
 template <typename T> __device__ __forceinline__ void stream_store(V2<T> *p, V2<T> x) { __builtin_nontemporal_store(x, p); }
 template <typename T> __device__ __forceinline__ void stream_store(__attribute__((address_space(1))) V2<T> *p, V2<T> x) {
     __builtin_nontemporal_store(x, p);
 }
+template <typename T, bool KEEP> __device__ __forceinline__ void flux_store(__attribute__((address_space(1))) V2<T> *p, V2<T> x) {
+    if constexpr (KEEP) *p = x;
+    else stream_store<T>(p, x);
+}
+
 // element v of a wavefront-uniform row: the row stays a scalar base and the lane adds a 32-bit byte offset
 template <typename T> __device__ __forceinline__ AS1 V2<T> *vslot(AS1 V2<T> *row, int v) {
     return (AS1 V2<T> *)((AS1 char *)row + (unsigned)v * (unsigned)sizeof(V2<T>));
@@ -777,7 +784,7 @@ template <typename T> constexpr bool kDeferStore = sizeof(T) == 8 ;
 // Velocity loop of one face through the tables.  WT: the normal runs along u
 // (the slow velocity index), else along v (the fast one).  mf collects the
 // macro flux sums.
-template <typename T, int M, bool WT>
+template <typename T, int M, bool WT, bool KEEP>
 __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, int lane,
                                                  AS3 char *tabN, AS3 char *tabT, AS1 V2<T> *fout, double (&mf)[4]) {
     const int NV = C.NV, nvt = __builtin_amdgcn_readfirstlane(C.nvt);
@@ -800,7 +807,7 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
         w = weight_at(C, v + 64 < NV ? v + 64 : v);
         stencil_load<T, M>(C, stn, v, delta, cur);
         if constexpr (kDeferStore<T>) {
-            if (v >= 64) stream_store<T>(vslot<T>(fout, v - 64), pend);
+            if (v >= 64) flux_store<T, KEEP>(vslot<T>(fout, v - 64), pend);
             last = v;
         }
         P2<T> ff, sg;
@@ -841,11 +848,11 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
             mf[3] = fma(0.5, fma(uu, X, ux * fma(SP2, s.hk * f0, th)), mf[3]);
         }
         if constexpr (kDeferStore<T>) pend = V2<T>{(T)rg, (T)rh};
-        else stream_store<T>(vslot<T>(fout, v), V2<T>{(T)rg, (T)rh});
+        else flux_store<T, KEEP>(vslot<T>(fout, v), V2<T>{(T)rg, (T)rh});
         ps += diu * ss; pf += djv * sf;
         if (pf >= pend_f) { pf -= nvt * sf; ps += ss; }
     }
-    if (last >= 0) stream_store<T>(vslot<T>(fout, last), pend);
+    if (last >= 0) flux_store<T, KEEP>(vslot<T>(fout, last), pend);
     if constexpr (sizeof(T) == 8) mf[3] *= 0.5;
 }
 
@@ -853,7 +860,7 @@ __device__ __forceinline__ void flux_loop_tables(const Consts &C, const Stencil<
 // velocities and polynomials formed per velocity.  On a tensor grid the FP64
 // plan's Maxwellian still factorises, in the global frame (its argument does
 // not depend on the frame): Ei[v / nvt] * Ej[v % nvt].
-template <typename T, int M>
+template <typename T, int M, bool KEEP>
 __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil<T> &stn, const FaceGeo &g, const FluxState &s, d2 n, int lane,
                                                   AS3 double *Ei, int nmax, AS1 V2<T> *fout, double (&mf)[4]) {
     const bool tensor = sizeof(T) == 8 && C.nut > 0;
@@ -882,7 +889,7 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
     face_velocity_loop<T, M>(C, stn, n, lane, vel, [&](int v, d2, d2 uv, int delta, const StenVals<T> &stv) __attribute__((always_inline)) {
         const double wv = vel.wc;
         if constexpr (kDeferStore<T>) {
-            if (v >= 64) stream_store<T>(fout + (v - 64), pend);
+            if (v >= 64) flux_store<T, KEEP>(fout + (v - 64), pend);
             last = v;
         }
         P2<T> ff, sg;
@@ -909,7 +916,7 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
         const double rg = ux * fma(f0, Bg + SP4, tg);
         const double rh = ux * fma(f0, fma(s.hk, Bg + SP2, fma(ux, Da, s.DT)), th);
         if constexpr (kDeferStore<T>) pend = V2<T>{(T)rg, (T)rh};
-        else stream_store<T>(fout + v, V2<T>{(T)rg, (T)rh});
+        else flux_store<T, KEEP>(fout + v, V2<T>{(T)rg, (T)rh});
         // macroFlux (clUGKS.c:607-661): the Shakhov and the non-equilibrium parts
         const double X = ux * fma(SP4, f0, tg);
         mf[0] += X;
@@ -917,10 +924,10 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
         mf[2] += uy * X;
         mf[3] += 0.5 * (uu * X + ux * fma(SP2, s.hk * f0, th));
     });
-    if (last >= 0) stream_store<T>(fout + last, pend);
+    if (last >= 0) flux_store<T, KEEP>(fout + last, pend);
 }
 
-template <typename T, int FW, int M>
+template <typename T, int FW, int M, bool KEEP>
 __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kFaceCWaves<T, M>))) k_faceC(const FBlock *__restrict__ blocks, const FaceRec *__restrict__ recs,
                                                    long long nfaces, const double *__restrict__ fstate, int nmax) {
     extern __shared__ __attribute__((aligned(16))) char fc_lds[];       // per wavefront: the tables
@@ -970,10 +977,10 @@ __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kF
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (wtype) flux_loop_tables<T, M, true>(C, stn, g, s, lane, tabN, tabT, fout, mf);
-        else flux_loop_tables<T, M, false>(C, stn, g, s, lane, tabN, tabT, fout, mf);
+        if (wtype) flux_loop_tables<T, M, true, KEEP>(C, stn, g, s, lane, tabN, tabT, fout, mf);
+        else flux_loop_tables<T, M, false, KEEP>(C, stn, g, s, lane, tabN, tabT, fout, mf);
     } else {
-        flux_loop_general<T, M>(C, stn, g, s, n, lane, (AS3 double *)tab, nmax, fout, mf);
+        flux_loop_general<T, M, KEEP>(C, stn, g, s, n, lane, (AS3 double *)tab, nmax, fout, mf);
     }
     wave_sum4(mf);
     if (lane == 0) {
@@ -1857,6 +1864,7 @@ struct ugks_step_plan {
     long long *d_face_off, *d_cell_off, *d_all_off;   // prefix offsets: interior faces, cells, all cells
     long long *d_tile_off;                              // prefix offsets of the update's 2 x 2 cell tiles
     long long nall, ntiles;
+    long long flux_bytes;                 // face fluxes of a step (interior faces)
     int nmax;                             // velocities on the longest axis of any block's tensor grid (at most 64)
     int fa_waves, fc_waves;               // workgroup size of the face passes, in wavefronts (1, 2 or 4)
     int method;                           // the blocks' common reconstruction method, -1 if they differ
@@ -1883,13 +1891,21 @@ struct ugks_step_plan {
 };
 
 namespace {
+// Ordinary stores for the face fluxes while the step's f and fluxes, three
+// arrays of about this size, stay in the 256 MB last-level cache; past the
+// caches beyond.  Step with ordinary / streaming stores on 2 x 2 blocks of n^2
+// (WENO5, 33^2 velocities): FP64 n = 24 (80 MB of fluxes) 157 / 163 us, n = 32
+// (143 MB) 230 / 233, n = 40 (223 MB) 360 / 330; mixed n = 24 (40 MB) 134 / 140,
+// n = 40 (112 MB) 244 / 259, n = 48 (161 MB) 325 / 321, n = 56 (219 MB) 438 / 417.
+constexpr long long kKeepFluxBytes = 144LL << 20;
 template <typename T, int FW, int M> void launch_faceA(ugks_step_plan *p, hipStream_t s) {
     hipLaunchKernelGGL((k_faceA<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
                        FW * (kAxisBytes * p->nmax), s, p->d_blocks, (const FaceRec *)p->d_frec,
                        p->nfaces, p->d_fsum, p->nmax);
 }
 template <typename T, int FW, int M> void launch_faceC(ugks_step_plan *p, hipStream_t s) {
-    hipLaunchKernelGGL((k_faceC<T, FW, M>), dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
+    auto *kernel = p->flux_bytes <= kKeepFluxBytes ? k_faceC<T, FW, M, true> : k_faceC<T, FW, M, false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((p->nfaces + FW - 1) / FW)), dim3(64 * FW),
                        FW * kTabBytes * p->nmax, s, p->d_blocks, (const FaceRec *)p->d_frec, p->nfaces,
                        (const double *)p->d_fstate, p->nmax);
 }
@@ -2190,6 +2206,8 @@ int ugks_step_plan_create_batch(ugks_block *const *blocks, const ugks_block_buff
         if (p->host_blocks[b].c.nut > 64 || p->host_blocks[b].c.nvt > 64) {
             delete p; return ugks_rt::fail(-2, "step plan: more than 64 velocities per axis");
         } else p->nmax = std::max(p->nmax, std::max(p->host_blocks[b].c.nut, p->host_blocks[b].c.nvt));
+    for (int b = 0; b < nblocks; b++)
+        p->flux_bytes += (face_off[b + 1] - face_off[b]) * p->host_blocks[b].c.NV * (precision == UGKS_FP64 ? 16 : 8);
     p->nfaces = face_off[nblocks];
     if (p->nfaces >= (1LL << 31)) { delete p; return ugks_rt::fail(-2, "step plan: 2^31 or more interior faces"); }
     p->ncells = cell_off[nblocks];
@@ -2598,6 +2616,8 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
             return ugks_rt::fail(-2, "step noalloc: more than 64 velocities per axis");
         else P.nmax = std::max(P.nmax, std::max(host[b].c.nut, host[b].c.nvt));
     if (T.off[0][nblocks] >= (1LL << 31)) return ugks_rt::fail(-2, "step noalloc: 2^31 or more interior faces");
+    for (int b = 0; b < nblocks; b++)
+        P.flux_bytes += (T.off[0][b + 1] - T.off[0][b]) * host[b].c.NV * (precision == UGKS_FP64 ? 16 : 8);
     P.npt = npt;
     P.nfaces = T.off[0][nblocks];
     P.ncells = T.off[1][nblocks];

@@ -39,3 +39,29 @@ def test_joint_launches_are_bitwise_the_separate_ones(hip, ncases, precision):
                 assert np.array_equal(x, y), name
     pj.close()
     pa.close()
+
+
+@pytest.mark.parametrize("precision,copies", [("fp64", 3), ("mixed", 6)])
+@pytest.mark.parametrize("method", ["WENO5", "vanLeer", "minmod"])
+@pytest.mark.parametrize("bent", [False, True])
+def test_kept_and_streamed_fluxes_are_bitwise_alike(hip, bent, method, precision, copies):
+    """A case alone keeps its 56 MB (28 in mixed mode) of face fluxes in the
+    caches; a plan of copies has more than 144 MB and streams them.  The stores
+    differ, the values do not."""
+    from pyugks_amd.fused import StepPlan
+    from pyugks_amd.sim import UGKSim
+    print(f"[gpu] flux stores {method} bent={bent} {precision}", flush=True)
+    g = cases.cavity(40, ("NC", 32), method, 0.05, n_cells_j=41, rho_perturb=0.01)
+    if bent:
+        cases.curvilinear(g, 0.05)
+    one, many = UGKSim(copy.deepcopy(g)), [UGKSim(copy.deepcopy(g)) for _ in range(copies)]
+    pairs = 2 * 40 * 41 * 33 * 33 * (16 if precision == "fp64" else 8)
+    assert pairs < 144 << 20 < copies * pairs * 39 / 40
+    po, pm = StepPlan(one, precision), StepPlan(many, precision)
+    po.run(3)
+    pm.run(3)
+    for sim in (many[0], many[-1]):
+        for name in ("macro_D", "Q_D", "wall_fluxes_D"):
+            assert np.array_equal(getattr(one.blocks[0], name).download(), getattr(sim.blocks[0], name).download()), name
+    po.close()
+    pm.close()
