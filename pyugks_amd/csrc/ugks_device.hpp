@@ -177,13 +177,16 @@ __device__ __forceinline__ double relax_time_of(const Consts &C, double base, do
 __device__ __forceinline__ double relax_time(const Consts &C, d4 p) { return relax_time_of(C, C.Kn / p.s0, p.s3); }
 
 // fM (clFunctions.c:49-58): weighted Maxwellian (g, h)
-__device__ __forceinline__ d2 maxwell(const Consts &C, d4 p, d2 uv, int v) {
+__device__ __forceinline__ double maxwell_g(d4 p, d2 uv) {
     double cx = uv.x - p.s1, cy = uv.y - p.s2;
-    double g = p.s0 * (p.s3 / kPi) * exp(-p.s3 * (cx * cx + cy * cy));
+    return p.s0 * (p.s3 / kPi) * exp(-p.s3 * (cx * cx + cy * cy));
+}
+__device__ __forceinline__ d2 maxwell_pair(const Consts &C, d4 p, double g, int v) {
     double h = (g * C.K) / (2.0 * p.s3);
     double w = C.weight[v];
     return d2{w * g, w * h};
 }
+__device__ __forceinline__ d2 maxwell(const Consts &C, d4 p, d2 uv, int v) { return maxwell_pair(C, p, maxwell_g(p, uv), v); }
 // fS (clFunctions.c:64-77): Shakhov correction of a Maxwellian M
 __device__ __forceinline__ d2 shakhov(const Consts &C, d4 p, d2 Q, d2 uv, d2 M) {
     double cx = uv.x - p.s1, cy = uv.y - p.s2;

@@ -136,19 +136,34 @@ template <typename Item> __device__ __forceinline__ int find_item(const Item *it
 template <typename T> __device__ __forceinline__ P2<T> ld(const void *p, size_t k) { return ((const P2<T> *)p)[k]; }
 template <typename T> __device__ __forceinline__ void st(void *p, size_t k, T x, T y) { ((P2<T> *)p)[k] = P2<T>{x, y}; }
 
-// ---- block-wide sum of N doubles (every thread receives the totals) --------
-template <int N> __device__ __forceinline__ void block_sum(double (&a)[N], double (*red)[16]) {
+// A double kept in the bits of a pair (x, y).  The empty asm keeps the two
+// words apart: merged into one 64-bit access they send an array of pairs from
+// registers to LDS.
+__device__ __forceinline__ void hold_d(double m, double &x, double &) { x = m; }
+__device__ __forceinline__ void hold_d(double m, float &x, float &y) {
+    x = __uint_as_float(lo_d(m));
+    y = __uint_as_float(hi_d(m));
+    __asm__("" : "+v"(x), "+v"(y));
+}
+__device__ __forceinline__ double held_d(double x, double) { return x; }
+__device__ __forceinline__ double held_d(float x, float y) {
+    __asm__("" : "+v"(x), "+v"(y));
+    return pack_d(__float_as_uint(x), __float_as_uint(y));
+}
+
+// ---- block-wide sum of N <= 4 doubles (every thread receives the totals) ----
+// Through columns AT .. AT + N - 1 of red, which nothing else in the kernel
+// writes: one barrier.
+template <int N, int AT> __device__ __forceinline__ void block_sum(double (&a)[N], double (*red)[16]) {
+    double four[4] = {};
 #pragma unroll
-    for (int q = 0; q < N; q++) a[q] = wave_sum(a[q]);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int q = 0; q < N; q++) red[w][q] = a[q];
-    }
+    for (int q = 0; q < N; q++) four[q] = a[q];
+    const double r = wave_sum4_rows(four);
+    const int row = (threadIdx.x & 63) >> 4;
+    if ((threadIdx.x & 15) == 0 && row < N) red[threadIdx.x >> 6][AT + row] = r;
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < N; q++) a[q] = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
-    __syncthreads();
+    for (int q = 0; q < N; q++) a[q] = (red[0][AT + q] + red[1][AT + q]) + (red[2][AT + q] + red[3][AT + q]);
 }
 
 // ---- reconstruction (iFace, clUGKS.c:134-195) in precision T ---------------
@@ -286,12 +301,6 @@ __device__ __forceinline__ double weight_at(const Consts &C, int v) {
 __device__ __forceinline__ double uniform_d(double x) {
     const unsigned long long b = (unsigned long long)__double_as_longlong(x);
     const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b), hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-// lane k's double, held in scalar registers
-template <int K> __device__ __forceinline__ double lane_d(double x) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, K), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), K);
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 // the reciprocals go through an empty asm so the compiler cannot turn the
@@ -1000,13 +1009,18 @@ struct WallItem { int block, wall; long long start; };
 // with nothing to switch to.  Measured on the 64-case batch (41^2 velocities
 // at most): 1.10 -> 0.86 ms mixed, 1.20 -> 0.97 ms FP64 (36 bytes spilled).
 // Beyond 7 the spills grow and the pass is a negligible share of the step.
+// The chain is what a face costs (of 17,300 clocks on 9^2 velocities 7,100 were its
+// two reductions), so the sums go through cross-lane swaps and one LDS round
+// without a second barrier, the 12 last ones are finished by 12 threads, and a
+// diffuse wall keeps the exponential of its first turn for the second: 9.9 ->
+// 7.8 us on two blocks of 6 x 10 cells, 15.5 -> 13.1 on 64^2 (mixed), 199 -> 174
+// on 16 blocks of 128^2 (mixed).
 template <int NPT> constexpr int kWallWaves = NPT <= 7 ? 3 : 1;
 template <typename T, int NPT>
 __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, const WallItem *__restrict__ items, int nitems,
                                           long long item, const DtState *__restrict__ ds) {
     __shared__ double red[kWavesT][16];
     __shared__ P2<T> wd[NPT * kT];   // reflected distribution (clAdsorb.c:377) for the specular mirror lookup
-    __shared__ double sc[8];
     const WallItem W = items[find_item(items, nitems, item)];
     const FBlock &B = blocks[W.block];
     const Consts &C = B.c;
@@ -1023,6 +1037,7 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
     const FaceGeo g = face_geo(B, gi, gj, fid);
     const d2 n = B.normal[g.own * 2 + fid];
     const double L = B.side_length[g.own * 2 + fid];
+    d4 wall = B.wall_prop[(size_t)ci * 4 + face];
     // reconstruction at the wall face (iFace)
     P2<T> ff[NPT];
     const Stencil<T> stn = stencil<T>(C, B.f, g);
@@ -1035,7 +1050,6 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
             reconstruct<T>(C, stn, g, v, upwind(uv.x), ff[k], sgk);
         }
     }
-    d4 wall = B.wall_prop[(size_t)ci * 4 + face];
     {
         d2 wl = to_local(mk2(wall.s1, wall.s2), n);
         wall.s1 = wl.x; wall.s2 = wl.y;
@@ -1048,11 +1062,15 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
             const int v = threadIdx.x + kT * k;
             if (v < C.NV) {
                 d2 uv = face_velocity(C, v, n);
-                if (leaves_wall(uv.x, rot)) s[1] -= uv.x * maxwell(C, wall, uv, v).x;
-                else s[0] += uv.x * (double)ff[k].x;
+                if (leaves_wall(uv.x, rot)) {
+                    // the Maxwellian waits in the place of the value it replaces
+                    const double m = maxwell_g(wall, uv);
+                    s[1] -= uv.x * (C.weight[v] * m);
+                    hold_d(m, ff[k].x, ff[k].y);
+                } else s[0] += uv.x * (double)ff[k].x;
             }
         }
-        block_sum<2>(s, red);
+        block_sum<2, 0>(s, red);
         const double ratio = s[0] / s[1];
 #pragma unroll
         for (int k = 0; k < NPT; k++) {
@@ -1060,7 +1078,7 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
             if (v < C.NV) {
                 d2 uv = face_velocity(C, v, n);
                 if (leaves_wall(uv.x, rot)) {
-                    d2 m = ratio * maxwell(C, wall, uv, v);
+                    const d2 m = ratio * maxwell_pair(C, wall, held_d(ff[k].x, ff[k].y), v);
                     ff[k] = P2<T>{(T)m.x, (T)m.y};
                 }
             }
@@ -1098,7 +1116,7 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
                 wd[threadIdx.x + kT * k] = P2<T>{(T)((tg - ag) / uv.x), (T)((th - ah) / uv.x)};
             }
         }
-        block_sum<3>(s3, red);
+        block_sum<3, 0>(s3, red);
         const double r_init = s3[0], a_init = s3[1], adjusted = s3[2];
         double a_final = a_init, dvtheta = 0.0, des = 0.0;
         bool early = false;
@@ -1170,7 +1188,7 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
                     }
                 }
             }
-            block_sum<1>(o, red);
+            block_sum<1, 3>(o, red);
             ratio = reflected / o[0];
         }
         const int account = ((des_cov == 0.0) && (ads_cov > 0.0) && (reflected == 0.0)) ? 1 : 0;
@@ -1217,18 +1235,25 @@ __device__ __forceinline__ void wall_face(const FBlock *__restrict__ blocks, con
             m4[10 + o] += 0.5 * (u2 * fgs + fhs);
         }
     }
-    block_sum<12>(m4, red);
-    if (threadIdx.x == 0) {
-        d2 gl = to_global(mk2(m4[1], m4[2]), n);
-        (fid == SOUTH ? B.fmS : B.fmW)[g.own] = (dt * L) * mk4(m4[0], gl.x, gl.y, m4[3]);
-        double *o = B.wall_fluxes + ((size_t)ci * 4 + face) * 8;
+    // totals: row r of each wavefront has sums 3 r .. 3 r + 2
+    double t[3];
+    wave_sum_rows<3>(m4, t);
+    if ((threadIdx.x & 15) == 0) {
+        const int row = (threadIdx.x & 63) >> 4;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            o[2 * q] = (double)(-rot) * m4[4 + 2 * q];
-            o[2 * q + 1] = (double)rot * m4[5 + 2 * q];
+        for (int k = 0; k < 3; k++) red[threadIdx.x >> 6][4 + 3 * row + k] = t[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 12) {
+        const int q = threadIdx.x;
+        auto total = [&](int c) { return (red[0][4 + c] + red[1][4 + c]) + (red[2][4 + c] + red[3][4 + c]); };
+        if (q == 0) {
+            const d2 gl = to_global(mk2(total(1), total(2)), n);
+            (fid == SOUTH ? B.fmS : B.fmW)[g.own] = (dt * L) * mk4(total(0), gl.x, gl.y, total(3));
+        } else if (q >= 4) {
+            B.wall_fluxes[((size_t)ci * 4 + face) * 8 + (q - 4)] = (double)(q & 1 ? rot : -rot) * total(q);
         }
     }
-    (void)sc;
 }
 
 // The wall faces and the state pass in one launch: neither fills the chip or
@@ -1371,25 +1396,25 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
         const double dW = ((((const double *)(B.fmS + c0))[k] - ((const double *)(B.fmS + c0 + 1))[k]) +
                            ((const double *)(B.fmW + c0))[k]) - ((const double *)(B.fmW + c0 + C.NJ))[k];
         r1 = (part < 4 ? dW : part == 4 ? 0.5 * pold.s0 : 1.0) / (part < 4 || part == 5 ? A : part == 4 ? pold.s3 : C.K);
-        const double w0 = pold.s0 + lane_d<0>(r1);
-        const double w1 = fma(pold.s0, pold.s1, lane_d<1>(r1)), w2 = fma(pold.s0, pold.s2, lane_d<2>(r1));
+        const double w0 = pold.s0 + lane_d(r1, 0);
+        const double w1 = fma(pold.s0, pold.s1, lane_d(r1, 1)), w2 = fma(pold.s0, pold.s2, lane_d(r1, 2));
         // u, v, 0.5 (w1^2 + w2^2) / rho; 0.5 rho / (gamma - 1) and the old state's 0.5 rho / lambda / (gamma - 1)
         const double r2 = (part == 0 ? w1 : part == 1 ? w2 : part == 2 ? 0.5 * fma(w1, w1, w2 * w2)
-                           : part == 3 ? 0.5 * w0 : lane_d<4>(r1)) / (part < 3 ? w0 : gm1);
-        const double e0 = fma(0.5 * pold.s0, fma(pold.s1, pold.s1, pold.s2 * pold.s2), lane_d<4>(r2));
-        const double w3 = e0 + lane_d<3>(r1);
+                           : part == 3 ? 0.5 * w0 : lane_d(r1, 4)) / (part < 3 ? w0 : gm1);
+        const double e0 = fma(0.5 * pold.s0, fma(pold.s1, pold.s1, pold.s2 * pold.s2), lane_d(r2, 4));
+        const double w3 = e0 + lane_d(r1, 3);
         p.s0 = w0;
-        p.s1 = lane_d<0>(r2);
-        p.s2 = lane_d<1>(r2);
-        p.s3 = lane_d<3>(r2) / (w3 - lane_d<2>(r2));
+        p.s1 = lane_d(r2, 0);
+        p.s2 = lane_d(r2, 1);
+        p.s3 = lane_d(r2, 3) / (w3 - lane_d(r2, 2));
         // even lanes the old state, odd lanes the new one
         const bool odd = lane & 1;
         const double rho = odd ? p.s0 : pold.s0, lam = odd ? p.s3 : pold.s3;
         const int q = part >> 1;
         r3 = (q == 0 ? C.Kn : q == 1 ? lam : q == 2 ? 0.8 * (1 - C.Pr) * (lam * lam) : C.K) /
              (q == 1 ? kPi : q == 3 ? 2.0 * lam : rho);
-        tau2 = relax_time_of(C, odd ? lane_d<1>(r3) : lane_d<0>(r3), lam);
-        rl = rho * (odd ? lane_d<3>(r3) : lane_d<2>(r3));
+        tau2 = relax_time_of(C, odd ? lane_d(r3, 1) : lane_d(r3, 0), lam);
+        rl = rho * (odd ? lane_d(r3, 3) : lane_d(r3, 2));
     }
     if (lane == 0) {
         B.macro_new[cell] = p;
@@ -1418,9 +1443,9 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const double pn1 = p.s1, pn2 = p.s2, pn3 = uniform_d(p.s3);
     const double Qx = uniform_d(Q.x), Qy = uniform_d(Q.y);
     const double ht = (0.5 * dt) / tau2;
-    const double uhto = lane_d<0>(ht), uhtn = lane_d<1>(ht), urden = uniform_d(1.0 / (1.0 + uhtn));
-    const double urlo = lane_d<0>(rl), urln = lane_d<1>(rl), uso = lane_d<4>(r3), usn = lane_d<5>(r3);
-    const double uhfo = lane_d<6>(r3), uhfn = lane_d<7>(r3), urA = lane_d<5>(r1), urK = lane_d<6>(r1);
+    const double uhto = lane_d(ht, 0), uhtn = lane_d(ht, 1), urden = uniform_d(1.0 / (1.0 + uhtn));
+    const double urlo = lane_d(rl, 0), urln = lane_d(rl, 1), uso = lane_d(r3, 4), usn = lane_d(r3, 5);
+    const double uhfo = lane_d(r3, 6), uhfn = lane_d(r3, 7), urA = lane_d(r1, 5), urK = lane_d(r1, 6);
     // this cell's velocities in f and in the four face fluxes: uniform bases, 32-bit lane offsets
     const long long NV = C.NV;
     AS1 V2<T> *fc = (AS1 V2<T> *)B.f + c0 * NV;
