@@ -287,6 +287,9 @@ template <typename T, bool KEEP> __device__ __forceinline__ void flux_store(__at
 template <typename T> __device__ __forceinline__ AS1 V2<T> *vslot(AS1 V2<T> *row, int v) {
     return (AS1 V2<T> *)((AS1 char *)row + (unsigned)v * (unsigned)sizeof(V2<T>));
 }
+// the same pointer, known to be to global memory: loads through it wait on the
+// vector-memory counter alone, in order
+template <typename P> __device__ __forceinline__ P *global_ptr(P *p) { return (P *)(AS1 P *)p; }
 // velocity table reads through global (not generic) pointers: they count only
 // against the vector-memory counter, so waiting for them does not also wait on LDS
 __device__ __forceinline__ d2 quad_at(const Consts &C, int v) {
@@ -1372,6 +1375,33 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const int gi = mi + C.G, gj = mj + C.G;
     const size_t c0 = (size_t)gi * C.NJ + gj;
     const double dt = ds[B.cs].dt_up;
+    const double A = *global_ptr(B.area + c0);
+    const d4 pold = *global_ptr(B.macro + cell);
+    const d2 Q = *global_ptr(B.qnext + cell);
+    const int k4 = lane & 3;
+    const double mS = *global_ptr((const double *)(B.fmS + c0) + k4), mN = *global_ptr((const double *)(B.fmS + c0 + 1) + k4);
+    const double mW = *global_ptr((const double *)(B.fmW + c0) + k4), mE = *global_ptr((const double *)(B.fmW + c0 + C.NJ) + k4);
+    // this cell's velocities in f and in the four face fluxes: uniform bases, 32-bit lane offsets
+    const long long NV = C.NV;
+    AS1 V2<T> *fc = (AS1 V2<T> *)B.f + c0 * NV;
+    AS1 V2<T> *fS = (AS1 V2<T> *)B.fluxS + c0 * NV, *fN = fS + NV;
+    AS1 V2<T> *fW = (AS1 V2<T> *)B.fluxW + c0 * NV, *fE = fW + (long long)C.NJ * NV;
+    struct Rows { V2<T> f, S, N, W, E; };
+    auto rows_at = [&](int v) { return Rows{*vslot<T>(fc, v), *vslot<T>(fS, v), *vslot<T>(fN, v), *vslot<T>(fW, v), *vslot<T>(fE, v)}; };
+    // FP64: the first turn's loads travel while the cell's constants are formed
+    // (64^2: 32.6 -> 30.6 us).  In mixed mode their registers would cost two of the
+    // seven wavefronts per SIMD (16 blocks of 128^2: 1.58 ms instead of 1.53), so
+    // they start behind the constants there.
+    Rows first{};
+    d2 enext = d2{0.0, 0.0};
+    double wnext = 0.0;
+    auto load_first = [&]() {
+        if (lane >= NV) return;
+        enext = quad_at(C, lane);
+        wnext = weight_at(C, lane);
+        first = rows_at(lane);
+    };
+    if constexpr (sizeof(T) == 8) load_first();
     // updateMacro (clUGKS.c:1158-1187) and the constants of UGKS_update
     // (:1189-1257).  All of it is the same for the wavefront's 64 lanes, and
     // most of it is divisions and a power: those that do not wait for one
@@ -1383,18 +1413,14 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     // 26.7 us; the FP64 one, bound by its bytes, stayed as it was.
     // Each operation rounds by itself (contraction off), but for the FMAs that
     // the conserved state takes the flux difference in.
-    const double A = B.area[c0], gm1 = C.gam - 1.0;
-    const d4 pold = B.macro[cell];
-    const d2 Q = B.qnext[cell];
+    const double gm1 = C.gam - 1.0;
     const int part = lane & 7;
     d4 p;
     double rl, tau2, r1, r3;
     {
 #pragma clang fp contract(off)
         // dW / A of component k in lane k, 0.5 rho / lambda in 4, 1 / A in 5, 1 / K in 6
-        const int k = lane & 3;
-        const double dW = ((((const double *)(B.fmS + c0))[k] - ((const double *)(B.fmS + c0 + 1))[k]) +
-                           ((const double *)(B.fmW + c0))[k]) - ((const double *)(B.fmW + c0 + C.NJ))[k];
+        const double dW = ((mS - mN) + mW) - mE;
         r1 = (part < 4 ? dW : part == 4 ? 0.5 * pold.s0 : 1.0) / (part < 4 || part == 5 ? A : part == 4 ? pold.s3 : C.K);
         const double w0 = pold.s0 + lane_d(r1, 0);
         const double w1 = fma(pold.s0, pold.s1, lane_d(r1, 1)), w2 = fma(pold.s0, pold.s2, lane_d(r1, 2));
@@ -1437,8 +1463,9 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     // the per-cell constants of the velocity loop in scalar registers, and one
     // 32-bit lane offset for the five rows: 71 VGPRs (seven waves per SIMD) in
-    // mixed mode, 81 in FP64 (five; held to 80 for six, 2 x 2 blocks of 128^2 took
-    // 969 us instead of 963, the channel 6.05 ms instead of 5.98)
+    // mixed mode, 91 in FP64 (five; six, at 80 VGPRs and without the early loads,
+    // took 969 us instead of 963 on 2 x 2 blocks of 128^2, 6.05 ms instead of 5.98
+    // on the channel)
     const double po1 = uniform_d(pold.s1), po2 = uniform_d(pold.s2), po3 = uniform_d(pold.s3);
     const double pn1 = p.s1, pn2 = p.s2, pn3 = uniform_d(p.s3);
     const double Qx = uniform_d(Q.x), Qy = uniform_d(Q.y);
@@ -1446,11 +1473,6 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     const double uhto = lane_d(ht, 0), uhtn = lane_d(ht, 1), urden = uniform_d(1.0 / (1.0 + uhtn));
     const double urlo = lane_d(rl, 0), urln = lane_d(rl, 1), uso = lane_d(r3, 4), usn = lane_d(r3, 5);
     const double uhfo = lane_d(r3, 6), uhfn = lane_d(r3, 7), urA = lane_d(r1, 5), urK = lane_d(r1, 6);
-    // this cell's velocities in f and in the four face fluxes: uniform bases, 32-bit lane offsets
-    const long long NV = C.NV;
-    AS1 V2<T> *fc = (AS1 V2<T> *)B.f + c0 * NV;
-    AS1 V2<T> *fS = (AS1 V2<T> *)B.fluxS + c0 * NV, *fN = fS + NV;
-    AS1 V2<T> *fW = (AS1 V2<T> *)B.fluxW + c0 * NV, *fE = fW + (long long)C.NJ * NV;
     // tensor indices of v = lane + 64 k, advanced without integer division
     int iu = 0, jv = 0, diu = 0, djv = 0;
     // the grid width in a register: the flux stores could alias the block
@@ -1462,10 +1484,8 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
     // the velocity and weight of the next iteration are loaded one iteration
     // ahead, and this velocity's f and face fluxes before its Maxwellians, so
     // the loads of an iteration overlap its arithmetic instead of stalling it
-    d2 enext = lane < C.NV ? quad_at(C, lane) : d2{0.0, 0.0};
-    double wnext = lane < C.NV ? weight_at(C, lane) : 0.0;
-    for (int v = lane; v < C.NV; v += 64) {
-        const V2<T> fo = *vslot<T>(fc, v), sS = *vslot<T>(fS, v), nS_ = *vslot<T>(fN, v), wW = *vslot<T>(fW, v), eW = *vslot<T>(fE, v);
+    auto turn = [&](int v, const Rows &r) {
+        const V2<T> fo = r.f, sS = r.S, nS_ = r.N, wW = r.W, eW = r.E;
         const d2 e = enext;
         const double w = wnext;
         {   // the next velocity's table entries (this one's again on the last round: no branch)
@@ -1502,7 +1522,10 @@ __global__ void __launch_bounds__(kT) k_update(const FBlock *__restrict__ blocks
         // the new cell's moments and heat flux (the next step's getAL / getAR and update inputs)
         add_moments<T>(e, tg, th, mom);
         add_heat<T>(nx, ny, cn, urK, tg, th, heat);
-    }
+    };
+    if constexpr (sizeof(T) == 4) load_first();
+    if (lane < NV) turn(lane, first);
+    for (int v = lane + 64; v < C.NV; v += 64) turn(v, rows_at(v));
     if (nan_seen) B.flag[0] = ERR_NAN;
     store_moments(B.cmom + c0, mom, lane);
     store_heat(B.qnext + cell, heat, lane);
