@@ -540,7 +540,7 @@ __device__ __forceinline__ FaceLoc face_loc_tiled(const FBlock &B, long long loc
 // One interior face as the face passes see it (64 bytes, one scalar load):
 // its block, side (SOUTH / WEST), owner cell and the reconstruction
 // distances of both upwind choices.  The plan fills the table from the mesh
-// (k_facerec) at every run call, so a geometry update under a live plan is
+// (k_refresh) at every run call, so a geometry update under a live plan is
 // picked up; the face passes then neither search the block offsets nor
 // recompute distances per face.
 struct __align__(64) FaceRec {
@@ -739,7 +739,7 @@ constexpr int kTabBytes = kTabN + kTabT;          // LDS bytes per wavefront and
 __device__ __forceinline__ V2<double> lpair(const AS3 char *p) { return *(const AS3 V2<double> *)p; }
 __device__ __forceinline__ void put_pair(AS3 char *p, double x, double y) { *(AS3 V2<double> *)p = V2<double>{x, y}; }
 
-// the face's folded flux constants (k_faceS)
+// the face's folded flux constants (face_state)
 struct FluxState {
     double U, V, lam, hk;
     d4 QL, QR, QT;
@@ -1003,7 +1003,7 @@ __global__ void __launch_bounds__(64 * FW) __attribute__((amdgpu_waves_per_eu(kF
     }
 }
 
-// ============================================================== k_wall ====
+// ============================================================== wall faces ====
 struct WallItem { int block, wall; long long start; };
 
 // Three waves per SIMD asked of the wall pass up to 7 velocities per thread
@@ -1282,7 +1282,7 @@ k_wallS(const FBlock *__restrict__ blocks, const WallItem *__restrict__ items, i
 // M = sum_v (g, e_x g, e_y g, (|e|^2 g + h) / 2) of one cell in the global
 // frame: the getAL/getAR moments of its faces after rotation into the face
 // frame.  Kept for every cell (ghosts included) by the update and the ghost
-// fill; k_cellmom recomputes them all at the start of each run.
+// fill; k_refresh recomputes them all at the start of each run.
 template <typename T>
 __device__ __forceinline__ void add_moments(d2 e, T gx, T hx, double (&m)[4]) {
     // The update (where g and h are products) and the refresh (where they are
@@ -1674,7 +1674,7 @@ __device__ __forceinline__ void join_corner(FBlock *blocks, int t) {
     F.flipidx[k] = flip;
 }
 
-// ============================================================ k_ghost ======
+// ============================================================ ghost cells ======
 struct GhostItem { int block, face; long long start; };
 
 template <typename T>
