@@ -2678,9 +2678,11 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
     P.nudf = T.nudf;
     P.udf_wl = udf_wl;
     // carve the working memory: 256-byte aligned regions, refused if they do not fit.
-    // A case's size is accounted with 128 bytes of face sums per face and no
-    // heat fluxes, so the same cases are taken as ever; the layout (96 or 104
-    // bytes per face and 16 per cell) is never larger where the limit is near.
+    // A case's size is accounted with 1168 bytes per block record, 128 bytes of
+    // face sums and 4 of a face index per face and no heat fluxes, so the same
+    // cases are taken as ever; the layout (a few bytes more per block, 96 or 104
+    // per face and 16 per cell) is never larger where the limit is near.
+    constexpr size_t kCountedRecord = 1168;
     size_t at = 0, counted = 0;
     auto carve = [&](size_t bytes, size_t as) {
         const size_t here = at;
@@ -2689,7 +2691,7 @@ int ugks_step_run_noalloc(ugks_block *const *blocks, const ugks_block_buffers *b
         return here;
     };
     auto region = [&](size_t bytes) { return carve(bytes, bytes); };
-    const size_t o_blocks = region(sizeof(FBlock) * nblocks), o_off = region(sizeof(long long) * 4 * (nblocks + 1)),
+    const size_t o_blocks = carve(sizeof(FBlock) * nblocks, kCountedRecord * nblocks), o_off = region(sizeof(long long) * 4 * (nblocks + 1)),
                  o_walls = region(sizeof(WallItem) * 4 * nblocks), o_ghosts = region(sizeof(GhostItem) * 4 * nblocks),
                  o_udf = region(sizeof(int) * nblocks), o_case = region(sizeof(int) * 3), o_state = region(sizeof(DtState)),
                  o_maxbits = region(sizeof(unsigned long long) * nblocks), o_maxdt = region(sizeof(double) * nblocks),
