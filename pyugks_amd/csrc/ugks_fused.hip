@@ -172,12 +172,15 @@ __device__ __forceinline__ float rcp_T(float x) { return __builtin_amdgcn_rcpf(x
 // WENO5 in FP32: the step from a stencil's middle cell to the face.  e_k =
 // 12 (eps + b_k) / sqrt(d_k) with the linear weights d = (0.1, 0.6, 0.3) riding
 // in the constants, and reciprocal estimates of the weights 1 / e_k^2.  Every
-// fused operation is written out: the results are rounded to FP32 again and
-// again, so the mixed plan keeps one order of operations whatever is built
-// around it.  (The FP64 form, weno5_q_pair in ugks_device.hpp, has fewer
-// operations, but would round every stored value of the mixed plan
-// differently.)  The passes specialised for WENO5 and the others (M = -1, and
-// the walls) fuse different terms of the middle candidate and of the sum.
+// fused operation is written out, so that the mixed plan's results do not
+// change with what is built around it.  That is a choice, not a need of its
+// accuracy: the FP64 form (weno5_q_pair in ugks_device.hpp) has fewer
+// operations and would round now and then a stored value the other way.  The
+// passes specialised for WENO5 and the others (M = -1, and the walls) fuse
+// different terms of the middle candidate and of the sum.  A mixed WENO5 case
+// that shares its plan with other limiters therefore differs from itself alone
+// in the last place of some stored values (after 3 steps of 24 x 20 cells: 5% of
+// f by at most 2e-7 of its maximum, rho, U, T by 1e-9, the heat flux by 4e-6).
 template <int M> __device__ __forceinline__ float weno5_f(float s0, float s1, float s2, float s3, float s4) {
     const float d1 = s1 - s0, d2 = s2 - s1, d3 = s3 - s2, d4 = s4 - s3;
     const float u0 = d2 - d1, v0 = fmaf(3.f, d2, -d1);
@@ -274,7 +277,6 @@ template <typename T> using V2 = T __attribute__((ext_vector_type(2)));
 // streams past the caches instead of evicting stencil data still in use.
 // KEEP: an ordinary store, for fluxes that stay in the 256 MB last-level cache
 // until the update reads them.
-template <typename T> __device__ __forceinline__ void stream_store(V2<T> *p, V2<T> x) { __builtin_nontemporal_store(x, p); }
 template <typename T> __device__ __forceinline__ void stream_store(__attribute__((address_space(1))) V2<T> *p, V2<T> x) {
     __builtin_nontemporal_store(x, p);
 }
@@ -487,9 +489,11 @@ __device__ __forceinline__ void face_velocity_loop(const Consts &C, const Stenci
 // needs the contracted third moment, which rotates as a vector, so no velocity
 // is rotated in the loop and 11 sums do.  The mixed plan's sums are the face
 // frame's, 0 g, 1 u g, 2 w g, 3 u^2 g, 4 w^2 g, 5 u w g, 6 u^3 g, 7 w^3 g,
-// 8 u w^2 g, 9 u^2 w g, 10 h, 11 u h, 12 w h: its f is rounded to FP32 every
-// step, where a last-bit difference in these sums would now and then turn a
-// stored value by one unit, so their order of operations is kept.
+// 8 u w^2 g, 9 u^2 w g, 10 h, 11 u h, 12 w h.  These sums are FP64 as well: their
+// order of operations is kept so that the mixed plan's results stay what they
+// were (see weno5_f), not for accuracy, and it costs instructions: 3.29e8 per
+// moment pass against the FP64 plan's 2.89e8 (2 x 2 blocks of 128^2 cells, 33^2
+// velocities).
 template <typename T> constexpr int kFS = sizeof(T) == 8 ? 12 : 13;   // face sums per face
 inline int kFSof(int precision) { return precision == UGKS_FP64 ? kFS<double> : kFS<float>; }
 constexpr int kFT = 32;                                               // face state per face
@@ -733,7 +737,8 @@ __device__ __forceinline__ void face_state(const FBlock *__restrict__ blocks, co
 // alone (T, 3 pairs).  A pair is one 16-byte LDS read; an odd number of pairs
 // per entry spreads consecutive entries over all banks.  The FP64 plan folds
 // everything that factorises; the mixed one keeps the order of operations of
-// the general loop (its flux is rounded to FP32, see the face sums).
+// the general loop (see the face sums): 3.90e8 instructions per flux pass against
+// 3.57e8 on the same case.
 constexpr int kTabN = 5 * 16, kTabT = 3 * 16;
 constexpr int kTabBytes = kTabN + kTabT;          // LDS bytes per wavefront and grid value of the longer axis
 __device__ __forceinline__ V2<double> lpair(const AS3 char *p) { return *(const AS3 V2<double> *)p; }
@@ -782,16 +787,20 @@ __device__ __forceinline__ void put_tangential(AS3 char *p, const FluxState &s, 
 }
 
 // minimum wavefronts per SIMD asked of the flux pass: the FP32 variants with a
-// fixed reconstruction run six (80 VGPRs; WENO5 spills 4 registers there and
-// is still faster than at five); the others are left to the compiler
+// fixed reconstruction run six (80 VGPRs, 1 or 2 of them spilled); the others
+// are left to the compiler.  With the tables the choice is level.  Flux pass at
+// six / five waves / the compiler's own: 2 x 2 blocks of 128^2 793 / 763 / 780 us,
+// 512^2 with 49^2 velocities 7.03 / 6.96 / 6.88 ms, 64^2 27 / 29 / 28 us, 200^2
+// vanLeer 401 / 425 / 466 us; steps within 1% but for the last (1.08 / 1.09 / 1.13 ms).
 template <typename T, int M> constexpr int kFaceCWaves = (sizeof(T) == 4 && M >= 0) ? 6 : 1;
 // The FP64 flux is stored one iteration late, so the wait for an iteration's
 // loads does not also wait for the store before them (the FP32 variant would
 // spill more at six waves).  Plain stencil loads: staged through LDS by
 // 16-byte LDS loads an iteration ahead, as this pass once did, the buffer costs
 // the waves that hide as much (uneven batch of 16 cases 3.65 -> 3.47 ms without
-// it, 64^2 cells 34.5 -> 32.4 us, 2 x 2 blocks of 128^2 level).
-template <typename T> constexpr bool kDeferStore = sizeof(T) == 8 ;
+// it, 64^2 cells 34.5 -> 32.4 us, 2 x 2 blocks of 128^2 level; in the general loop,
+// a bent grid of 200 x 190 cells with WENO5 and 33^2 velocities 850 -> 785 us).
+template <typename T> constexpr bool kDeferStore = sizeof(T) == 8;
 
 // Velocity loop of one face through the tables.  WT: the normal runs along u
 // (the slow velocity index), else along v (the fast one).  mf collects the
@@ -893,8 +902,8 @@ __device__ __forceinline__ void flux_loop_general(const Consts &C, const Stencil
     // record, so C.nvt would otherwise be loaded again in every iteration
     const int nvt = __builtin_amdgcn_readfirstlane(C.nvt);
     if (tensor) { iu = lane / nvt; jv = lane - iu * nvt; diu = 64 / nvt; djv = 64 - diu * nvt; }
-    // each velocity's flux is stored one iteration late, at the start of the
-    // next, so the wait for the loads issued there does not also wait for it
+    // in FP64 each velocity's flux is stored one iteration late, at the start of
+    // the next, so the wait for the loads issued there does not also wait for it
     V2<T> pend = V2<T>{T(0), T(0)};
     int last = -1;
     TableVelocities<true> vel(C, lane);
@@ -1707,7 +1716,7 @@ __device__ __forceinline__ void ghost_cell(const FBlock *__restrict__ blocks, co
     const size_t NV = C.NV;
     const size_t dst = ((size_t)gi * C.NJ + gj) * NV;
     const int type = B.bc[face];
-    // the ghost cell's moments for the faces it borders (uniform exits: the whole workgroup reaches these)
+    // the ghost cell's moments for the faces it borders (uniform exits: the whole wavefront reaches these)
     double m[4] = {0.0, 0.0, 0.0, 0.0};
     auto put = [&](int v, P2<T> x) {
         ((P2<T> *)B.f)[dst + v] = x;
@@ -1865,9 +1874,12 @@ __global__ void __launch_bounds__(kT) k_end(const FBlock *__restrict__ blocks, E
     cell_dt(blocks, e.cell_off, e.nb, e.ds, e.maxbits, g);
     // Only the maxima cross workgroups, and those are atomics at the device's
     // scope on both sides: it is enough that a wavefront's are performed before
-    // its workgroup draws a ticket.  A __threadfence() here would also write the
-    // L2 back per workgroup (16 blocks of 128^2: 195 us instead of 138 for the
-    // three launches).
+    // its workgroup draws a ticket.  That rests on gfx950, not on the language's
+    // memory model: an atomic without a result counts in vmcnt until it is
+    // performed where the device's scope asks, and the loads of case_dt, at that
+    // scope too, do not take a stale line.  A __threadfence() here would also
+    // write the L2 back per workgroup (16 blocks of 128^2: 195 us instead of 138
+    // for the three launches).
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) last = atomicAdd(e.ticket, 1u) == (unsigned)(e.ndt_groups - 1);
@@ -1939,9 +1951,9 @@ struct ugks_step_plan {
 };
 
 namespace {
-// Ordinary stores for the face fluxes while the step's f and fluxes, three
-// arrays of about this size, stay in the 256 MB last-level cache; past the
-// caches beyond.  Step with ordinary / streaming stores on 2 x 2 blocks of n^2
+// Ordinary stores for the face fluxes (both arrays together, interior faces)
+// up to this size: with f, half as large, they then fill 216 MB of the 256 MB
+// last-level cache at most; past the caches beyond.  Step with ordinary / streaming stores on 2 x 2 blocks of n^2
 // (WENO5, 33^2 velocities): FP64 n = 24 (80 MB of fluxes) 157 / 163 us, n = 32
 // (143 MB) 230 / 233, n = 40 (223 MB) 360 / 330; mixed n = 24 (40 MB) 134 / 140,
 // n = 40 (112 MB) 244 / 259, n = 48 (161 MB) 325 / 321, n = 56 (219 MB) 438 / 417.
@@ -2006,10 +2018,15 @@ template <typename T, int NPT> int launch_step(ugks_step_plan *p, hipStream_t s,
     if (p->nfaces > 0)
         faceA<T>(p, s, p->fa_waves);
     if (ev) (void)hipEventRecord(ev[1], s);
-    // Walls beside the states while they are few enough to be latency, not work:
-    // 9 us off a mixed step of 2 x 2 blocks of 128^2 (1,028 workgroups).  With 16 blocks of 128^2 (10,256) the launches take as long together
-    // as apart, and an update straight behind the flux pass takes longer than
-    // one behind the walls: 6.00 against 5.96 ms a step.
+    // Walls beside the states while they are few enough to be latency, not work.
+    // Step apart / beside (WENO5): 15 cases of 32^2 (2,037 workgroups) 253 / 247 us
+    // in FP64 and 197 / 190 mixed, 30 of them (4,073) 363 / 358 mixed.  From about
+    // 3,000 workgroups of larger cases on, both are level within what runs differ:
+    // 400^2 (2,847) 2.82 / 2.81 ms mixed, 512^2 with 17^2 velocities (4,092) 2.53 /
+    // 2.53, the channel with 25^2 (4,100) 4.54 / 4.54, 600^2 (5,208) 6.27 / 6.31.  With
+    // 16 blocks of 128^2 (10,224) apart is the faster mixed one (4.70 / 4.73): the
+    // launches take as long together as apart, and an update straight behind the
+    // flux pass takes longer than one behind the walls.
     const bool beside = !ev && p->nwalls + (p->nfaces + kT - 1) / kT <= 4096;
     launch_wallS<T, NPT>(p, s, beside ? p->nwalls : 0, p->nfaces);
     if (ev) (void)hipEventRecord(ev[2], s);
@@ -2080,8 +2097,8 @@ __host__ __device__ void flux_loop_dts(DtState &d, double M) {
 
 template <typename T> int autotune(ugks_step_plan *p, hipStream_t s, int reps, int32_t *choice) {
     // The face passes only read f and the step state and rewrite per-step scratch
-    // (face sums, face states, fluxes, Q from the same f), so timing them
-    // repeatedly leaves the simulation state as it was.
+    // (face sums, face states, fluxes), so timing them repeatedly leaves the
+    // simulation state as it was.
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
         return ugks_rt::fail(-1, "autotune: event create");

@@ -9,7 +9,10 @@ faces), with each case's time step kept on the device (one UGKSim.one_step per c
 With ``graph=True`` the step runs as replays of a captured HIP graph.  With
 ``precision="mixed"`` f and the per-velocity face fluxes are stored and
 computed in FP32; moments, the macroscopic update, heat fluxes, equilibrium
-moments and the time step stay FP64.
+moments and the time step stay FP64.  A case's results do not depend on the
+other cases of its plan, but for the rounding: where the plan holds several
+limiters, its face passes are the general ones, which round the mixed WENO5's
+FP32 values (and a few FP64 ones) in another order.
 """
 from __future__ import annotations
 
