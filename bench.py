@@ -112,11 +112,12 @@ def cpu_model():
 
 
 def read_profile_table(fname, workload):
-    """Per-launch figures {kernel: value} for one workload from a counter
-    summary committed under profiles/ (lines "kernel workload value ..."), and
-    the source commit the summary says it was measured on ("# source commit
-    <hash>").  These are NOT measured by this run: they are labelled with
-    their file and commit wherever they are reported."""
+    """Per-step figures {kernel: value} for one workload from a counter summary
+    committed under profiles/ (lines "kernel workload launches value ...", the
+    value added up over a kernel's launches in a step), and the source commit
+    the summary says it was measured on ("# source commit <hash>").  These are
+    NOT measured by this run: they are labelled with their file and commit
+    wherever they are reported."""
     path = os.path.join(ROOT, "profiles", fname)
     if not os.path.exists(path):
         return {}, None
@@ -127,11 +128,8 @@ def read_profile_table(fname, workload):
                 commit = line.split()[-1]
                 continue
             parts = line.split()
-            if len(parts) >= 3 and parts[1] == workload and not line.startswith("#"):
-                try:
-                    out[parts[0]] = float(parts[2])
-                except ValueError:
-                    pass
+            if len(parts) >= 4 and parts[1] == workload and not line.startswith("#"):
+                out[parts[0]] = float(parts[3])
     return out, commit
 
 
@@ -193,19 +191,15 @@ def run_precision(gs, precision, a, upd_per_step, workload):
     k_ach = b_alg * upd_per_step / (per_launch[dom] * 1e-3) / 1e9
     roof["dominant_kernel"] = {"kernel": dom, "ms_per_launch": per_launch[dom], "achieved": k_ach,
                                "frac": k_ach / HBM_PEAK_GBS}
-    # the launches of a step (not the per-call refresh): joined ones in a run, parts in the timed steps
-    step_kernels = set(per_launch) | {"k_wallS", "k_end"}
     traffic, t_commit = read_profile_table(f"hbm_traffic_per_kernel_{workload}.txt", tag)
-    traffic = {k: v for k, v in traffic.items() if k in step_kernels}
     if traffic:
         roof["traffic"] = sum(traffic.values())
         roof["traffic_source"] = (f"profiles/hbm_traffic_per_kernel_{workload}.txt, rocprofv3 FETCH_SIZE + "
-                                  f"WRITE_SIZE summed over the step's kernels, source commit {t_commit}")
+                                  f"WRITE_SIZE summed over the step's launches, source commit {t_commit}")
         roof["traffic_over_alg"] = roof["traffic"] / (b_alg * upd_per_step)
     else:
         roof["traffic"] = None
     valu, v_commit = read_profile_table(f"valu_per_kernel_{workload}.txt", tag)
-    valu = {k: v for k, v in valu.items() if k in step_kernels}
     if valu:
         per_step = sum(valu.values())
         roof["valu"] = {"insts_per_step": per_step,
