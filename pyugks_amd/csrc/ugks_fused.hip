@@ -1019,7 +1019,7 @@ struct WallItem { int block, wall; long long start; };
 // (NV <= 1792): the compiler's own choice, 170-184 VGPRs, leaves two, and the
 // pass, a chain of loads and workgroup reductions per wall face, then waits
 // with nothing to switch to.  Measured on the 64-case batch (41^2 velocities
-// at most): 1.10 -> 0.86 ms mixed, 1.20 -> 0.97 ms FP64 (36 bytes spilled).
+// at most): 1.10 -> 0.86 ms mixed, 1.20 -> 0.97 ms FP64 (36 bytes spilled, 12 now).
 // Beyond 7 the spills grow and the pass is a negligible share of the step.
 // The chain is what a face costs (of 17,300 clocks on 9^2 velocities 7,100 were its
 // two reductions), so the sums go through cross-lane swaps and one LDS round
